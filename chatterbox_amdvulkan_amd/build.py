@@ -36,6 +36,7 @@ SOURCES = [
     "k_softmax.hip",
     "k_norm_ext.hip",
     "k_conv1d.hip",
+    "k_resblock.hip",
     "k_eltwise.hip",
     "k_batch.hip",
     "k_binary.hip",

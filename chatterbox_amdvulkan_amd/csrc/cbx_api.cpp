@@ -1152,17 +1152,115 @@ static int check_conv_x(const char* what, const cbx_conv1d_weights* w, const cbx
     return CBX_OK;
 }
 
-// cbx_conv1d and cbx_conv1d_sum: acc (with its scale) only from the latter
-static int conv1d_common(const char* what, const cbx_tensor* x, const cbx_conv1d_weights* w, int stride, int pad,
-                         int dilation, int prologue, const cbx_tensor* alpha, const cbx_tensor* alpha_inv, float slope,
-                         const cbx_tensor* bias, const cbx_tensor* res, const cbx_tensor* acc, float scale,
-                         cbx_tensor* y, cbx_stream stream);
+extern "C++" {
+
+// Everything a cbx_conv1d / cbx_conv1d_sum call checks before it launches.
+static int check_conv1d(const char* what, const ConvCall& c, DeviceState** st, bool* empty) {
+    int rc;
+    *empty = false;
+    *st = current_state(&rc);
+    if (!*st) return rc;
+    if (!c.w) return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": weights are NULL");
+    if ((rc = validate(c.x, what, "x")) || (rc = validate(c.y, what, "y"))) return rc;
+    if ((rc = check_conv_x(what, c.w, c.x, c.prologue))) return rc;
+    if (c.stride < 1 || c.pad < 0 || c.dilation < 1 || c.stride > 64 || c.pad > (1 << 20) || c.dilation > 1024) {
+        return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": stride must be 1..64, pad >= 0, dilation 1..1024");
+    }
+    const int64_t t_in = c.x->ne[1];
+    const int64_t span = c.dilation * (c.w->k - 1) + 1;
+    const int64_t t_out = t_in + 2 * c.pad >= span ? (t_in + 2 * c.pad - span) / c.stride + 1 : 0;
+    if ((rc = check_conv_io(what, c.w, false, c.prologue, c.x, c.alpha, c.alpha_inv, c.bias, c.res, c.y, t_out,
+                            "T_out = (T_in + 2 pad - dilation (K - 1) - 1) / stride + 1", empty))) {
+        return rc;
+    }
+    if (*empty) return CBX_OK;
+    if (c.acc) {
+        if ((rc = validate(c.acc, what, "acc"))) return rc;
+        if (c.acc->type != CBX_TYPE_F32 || !same_shape(c.acc, c.y)) {
+            return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": acc must be F32 with y's shape");
+        }
+        // read in the epilogue while other workgroups store their tiles
+        if (overlaps(c.acc, c.y)) return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": acc must not overlap y");
+    }
+    return CBX_OK;
+}
+
+int cbx::conv1d_call(const ConvCall& c, cbx_stream stream) {
+    clear_error();
+    DeviceState* st = nullptr;
+    bool empty = false;
+    const int rc = check_conv1d(c.acc ? "cbx_conv1d_sum" : "cbx_conv1d", c, &st, &empty);
+    if (rc || empty) return rc;
+    const bool snake = c.prologue == CBX_CONV_PRO_SNAKE;
+    return launch_conv1d(c.x, c.w->data, c.w->k, c.w->c_in_pad, c.w->c_out, c.stride, c.pad, c.dilation, 1, 0, c.w->w_ph,
+                         c.prologue, snake ? c.alpha : nullptr, snake ? c.alpha_inv : nullptr, c.slope, c.bias, c.res,
+                         c.y, st, reinterpret_cast<hipStream_t>(stream), c.acc, c.scale);
+}
+
+// The one-launch form takes what both calls accept, at one batch item, with
+// every vector access aligned, and no output byte shared with an input: its
+// workgroups read x's halo rows while others store y (one by one, conv2 may
+// write over its residual).
+bool cbx::res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int* ch) {
+    if (!c1.w || !c2.w || c1.prologue != CBX_CONV_PRO_SNAKE || c2.prologue != CBX_CONV_PRO_SNAKE || c1.res || c1.acc ||
+        !c1.bias || !c2.bias || !c2.res || c1.y != c2.x || c1.stride != 1 || c2.stride != 1 ||
+        2 * static_cast<int64_t>(c1.pad) != (c1.w->k - 1) * c1.dilation ||
+        2 * static_cast<int64_t>(c2.pad) != (c2.w->k - 1) * c2.dilation || c1.w->c_in != c1.w->c_out ||
+        c2.w->c_in != c2.w->c_out || c1.w->c_in != c2.w->c_in) {
+        return false;
+    }
+    DeviceState* st = nullptr;
+    bool e1 = false, e2 = false;
+    if (check_conv1d("cbx_conv1d", c1, &st, &e1) || check_conv1d("cbx_conv1d", c2, &st, &e2) || e1 || e2) {
+        clear_error();   // the calls report it when they run one by one
+        return false;
+    }
+    if (c1.x->ne[2] != 1) return false;
+    auto rows16 = [](const cbx_tensor* t) {
+        return reinterpret_cast<uintptr_t>(t->data) % 16 == 0 && t->nb[1] % 16 == 0;
+    };
+    for (const cbx_tensor* t : {c1.x, static_cast<const cbx_tensor*>(c2.y), c2.res, c2.acc}) {
+        if (t && !rows16(t)) return false;
+    }
+    for (const cbx_tensor* t : {c1.alpha, c1.alpha_inv, c1.bias, c2.alpha, c2.alpha_inv, c2.bias}) {
+        if (reinterpret_cast<uintptr_t>(t->data) % 16 || overlaps(t, c2.y)) return false;
+    }
+    if (overlaps(c1.x, c2.y) || overlaps(c2.res, c2.y)) return false;
+    l->x = static_cast<const char*>(c1.x->data);
+    l->w1 = c1.w->data;
+    l->w2 = c2.w->data;
+    l->al1 = static_cast<const float*>(c1.alpha->data);
+    l->ai1 = static_cast<const float*>(c1.alpha_inv->data);
+    l->b1 = static_cast<const float*>(c1.bias->data);
+    l->al2 = static_cast<const float*>(c2.alpha->data);
+    l->ai2 = static_cast<const float*>(c2.alpha_inv->data);
+    l->b2 = static_cast<const float*>(c2.bias->data);
+    l->res = static_cast<const char*>(c2.res->data);
+    l->acc = c2.acc ? static_cast<const char*>(c2.acc->data) : nullptr;
+    l->y = static_cast<char*>(c2.y->data);
+    l->x_nb1 = static_cast<int64_t>(c1.x->nb[1]);
+    l->r_nb1 = static_cast<int64_t>(c2.res->nb[1]);
+    l->a_nb1 = c2.acc ? static_cast<int64_t>(c2.acc->nb[1]) : 0;
+    l->y_nb1 = static_cast<int64_t>(c2.y->nb[1]);
+    l->T = static_cast<int32_t>(c1.x->ne[1]);
+    l->k1 = static_cast<int32_t>(c1.w->k);
+    l->d1 = c1.dilation;
+    l->k2 = static_cast<int32_t>(c2.w->k);
+    l->d2 = c2.dilation;
+    l->scaled = c2.acc && c2.scale != 1.0f;
+    l->oscale = c2.scale;
+    l->tiles = 0;
+    *ch = static_cast<int>(c1.w->c_in);
+    return res_layer_fits(*l, *ch, st);
+}
+
+}  // extern "C++"
 
 int cbx_conv1d(const cbx_tensor* x, const cbx_conv1d_weights* w, int stride, int pad, int dilation, int prologue,
                const cbx_tensor* alpha, const cbx_tensor* alpha_inv, float slope, const cbx_tensor* bias,
                const cbx_tensor* res, cbx_tensor* y, cbx_stream stream) {
-    return conv1d_common("cbx_conv1d", x, w, stride, pad, dilation, prologue, alpha, alpha_inv, slope, bias, res,
-                         nullptr, 1.0f, y, stream);
+    return conv1d_call(ConvCall{x, w, stride, pad, dilation, prologue, alpha, alpha_inv, slope, bias, res, nullptr, 1.0f, y},
+                       stream);
 }
 
 int cbx_conv1d_sum(const cbx_tensor* x, const cbx_conv1d_weights* w, int stride, int pad, int dilation, int prologue,
@@ -1172,45 +1270,8 @@ int cbx_conv1d_sum(const cbx_tensor* x, const cbx_conv1d_weights* w, int stride,
         clear_error();
         return set_error(CBX_ERR_INVALID_ARG, "cbx_conv1d_sum: acc is NULL (cbx_conv1d has no sum)");
     }
-    return conv1d_common("cbx_conv1d_sum", x, w, stride, pad, dilation, prologue, alpha, alpha_inv, slope, bias, res,
-                         acc, scale, y, stream);
-}
-
-static int conv1d_common(const char* what, const cbx_tensor* x, const cbx_conv1d_weights* w, int stride, int pad,
-                         int dilation, int prologue, const cbx_tensor* alpha, const cbx_tensor* alpha_inv, float slope,
-                         const cbx_tensor* bias, const cbx_tensor* res, const cbx_tensor* acc, float scale,
-                         cbx_tensor* y, cbx_stream stream) {
-    clear_error();
-    int rc;
-    DeviceState* st = current_state(&rc);
-    if (!st) return rc;
-    if (!w) return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": weights are NULL");
-    if ((rc = validate(x, what, "x")) || (rc = validate(y, what, "y"))) return rc;
-    if ((rc = check_conv_x(what, w, x, prologue))) return rc;
-    if (stride < 1 || pad < 0 || dilation < 1 || stride > 64 || pad > (1 << 20) || dilation > 1024) {
-        return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": stride must be 1..64, pad >= 0, dilation 1..1024");
-    }
-    const int64_t t_in = x->ne[1];
-    const int64_t span = dilation * (w->k - 1) + 1;
-    const int64_t t_out = t_in + 2 * pad >= span ? (t_in + 2 * pad - span) / stride + 1 : 0;
-    bool empty = false;
-    if ((rc = check_conv_io(what, w, false, prologue, x, alpha, alpha_inv, bias, res, y, t_out,
-                            "T_out = (T_in + 2 pad - dilation (K - 1) - 1) / stride + 1", &empty))) {
-        return rc;
-    }
-    if (empty) return CBX_OK;
-    if (acc) {
-        if ((rc = validate(acc, what, "acc"))) return rc;
-        if (acc->type != CBX_TYPE_F32 || !same_shape(acc, y)) {
-            return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": acc must be F32 with y's shape");
-        }
-        // read in the epilogue while other workgroups store their tiles
-        if (overlaps(acc, y)) return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": acc must not overlap y");
-    }
-    return launch_conv1d(x, w->data, w->k, w->c_in_pad, w->c_out, stride, pad, dilation, 1, 0, w->w_ph, prologue,
-                         prologue == CBX_CONV_PRO_SNAKE ? alpha : nullptr,
-                         prologue == CBX_CONV_PRO_SNAKE ? alpha_inv : nullptr, slope, bias, res, y, st,
-                         reinterpret_cast<hipStream_t>(stream), acc, scale);
+    return conv1d_call(ConvCall{x, w, stride, pad, dilation, prologue, alpha, alpha_inv, slope, bias, res, acc, scale, y},
+                       stream);
 }
 
 int cbx_conv_transpose1d(const cbx_tensor* x, const cbx_conv1d_weights* w, int pad, int prologue,

@@ -897,6 +897,79 @@ constexpr int32_t kSpan[][2] = {
 constexpr int32_t kLastKind = CBX_GL_ROPE_TWO;
 static_assert(sizeof(kSpan) / sizeof(kSpan[0]) == kLastKind + 1, "one span per launch kind");
 
+constexpr int kConvMisfit = 1;   // conv_call_of: the launch does not fit the node list
+
+// The call a CONV1D or CONV_TRANSPOSE1D launch (its span inside the node
+// list) makes: the layout its flags describe -- prologue, body, bias,
+// residual [, the sum [, its scale]].  For the transposed conv c->pad is the
+// crop.
+int conv_call_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, ConvCall* c) {
+    const int32_t f = l.first_node;
+    const cbx_gnode& a = nd[f];
+    const int pro = l.flags & 3;
+    const bool bias = (l.flags & 4) != 0, res = (l.flags & 8) != 0;
+    const bool sum = (l.flags & 16) != 0, scl = (l.flags & 32) != 0;
+    const bool tr = l.kind == CBX_GL_CONV_TRANSPOSE1D;
+    const int32_t p = pro == 1 ? 5 : pro == 2 ? 1 : 0;
+    const int32_t n_res = p + (tr ? 7 : 9) + (bias ? 2 : 0) + (res ? 1 : 0);   // nodes up to the residual add
+    if (pro == 3 || (tr && (res || sum)) || (sum && !res) || (scl && !sum) ||
+        l.n_nodes != n_res + (sum ? 1 : 0) + (scl ? 1 : 0)) {
+        return kConvMisfit;
+    }
+    const int32_t b0 = f + p;   // the transpose view
+    c->x = T(t, a.src[0]);
+    c->y = const_cast<cbx_tensor*>(&t[nd[f + l.n_nodes - 1].dst]);
+    c->alpha = pro == 1 ? T(t, a.src[1]) : nullptr;
+    c->alpha_inv = pro == 1 ? T(t, nd[f + 3].src[1]) : nullptr;
+    c->slope = pro == 2 ? a.fparam : 0.0f;
+    c->prologue = pro == 1 ? CBX_CONV_PRO_SNAKE : pro == 2 ? CBX_CONV_PRO_LEAKY_RELU : CBX_CONV_PRO_NONE;
+    const int32_t bview = b0 + (tr ? 5 : 7);   // the bias view, when there is one
+    c->bias = bias ? T(t, nd[bview].src[0]) : nullptr;
+    c->res = c->acc = nullptr;
+    c->scale = 1.0f;
+    c->stride = c->dilation = 1;
+    // the prepared weights must be the node's weight tensor's
+    const cbx_gnode& wn = nd[b0 + (tr ? 2 : 5)];
+    const cbx_tensor* wk = T(t, nd[b0 + 2].src[0]);
+    if (!wk || !conv1d_weights_match(wn.conv_w, tr ? wn.conv[0] : 0, wk->ne[0], tr ? wk->ne[2] : wk->ne[1],
+                                     tr ? wk->ne[1] : wk->ne[2])) {
+        return set_error(CBX_ERR_INVALID_ARG, "cbx_graph_launch: node " + std::to_string(b0 + (tr ? 2 : 5)) +
+                                                  ": conv_w was not made from the node's weight tensor");
+    }
+    c->w = wn.conv_w;
+    if (!tr) {
+        const cbx_gnode& ic = nd[b0 + 2];
+        c->stride = ic.conv[0];
+        c->pad = ic.conv[1];
+        c->dilation = ic.conv[2];
+        if (res) {
+            const cbx_gnode& ra = nd[f + n_res - 1];   // add(residual, conv out)
+            const int32_t out = nd[f + n_res - 2].dst;
+            c->res = T(t, ra.src[0] == out ? ra.src[1] : ra.src[0]);
+        }
+        if (!sum) return CBX_OK;
+        const cbx_gnode& sa = nd[f + n_res];          // add(acc, residual's result)
+        const int32_t rr = nd[f + n_res - 1].dst;
+        if (sa.op != CBX_GOP_ADD || (sa.src[0] != rr && sa.src[1] != rr)) return kConvMisfit;
+        c->acc = T(t, sa.src[0] == rr ? sa.src[1] : sa.src[0]);
+        if (!c->acc) return kConvMisfit;
+        if (scl) {
+            const cbx_gnode& sn = nd[f + n_res + 1];
+            if (sn.op != CBX_GOP_SCALE || sn.src[0] != sa.dst) return kConvMisfit;
+            c->scale = sn.fparam;
+        }
+        return CBX_OK;
+    }
+    // the crop: the view's offset into the full output, in frames
+    const cbx_tensor* full = T(t, nd[b0 + 2].dst);
+    const cbx_tensor* crop = T(t, nd[b0 + 3].dst);
+    if (!full || !crop) return kConvMisfit;
+    const int64_t off = static_cast<const char*>(crop->data) - static_cast<const char*>(full->data);
+    if (off < 0 || off % 4 || off / 4 > (int64_t{1} << 30)) return kConvMisfit;
+    c->pad = static_cast<int>(off / 4);
+    return CBX_OK;
+}
+
 // Issues the entry point a launch maps to.  A launch is only read within
 // the node list, so one not made by the planner cannot read past it.
 int run(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const cbx_glaunch& l, cbx_stream s) {
@@ -1124,66 +1197,12 @@ int run(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const cbx_gla
         }
         case CBX_GL_CONV1D:
         case CBX_GL_CONV_TRANSPOSE1D: {
-            // the layout the flags describe: prologue, body, bias, residual
-            // [, the sum [, its scale]]
-            const int pro = l.flags & 3;
-            const bool bias = (l.flags & 4) != 0, res = (l.flags & 8) != 0;
-            const bool sum = (l.flags & 16) != 0, scl = (l.flags & 32) != 0;
-            const bool tr = l.kind == CBX_GL_CONV_TRANSPOSE1D;
-            const int32_t p = pro == 1 ? 5 : pro == 2 ? 1 : 0;
-            const int32_t n_res = p + (tr ? 7 : 9) + (bias ? 2 : 0) + (res ? 1 : 0);   // nodes up to the residual add
-            if (pro == 3 || (tr && (res || sum)) || (sum && !res) || (scl && !sum) ||
-                l.n_nodes != n_res + (sum ? 1 : 0) + (scl ? 1 : 0)) {
-                break;
-            }
-            const int32_t b0 = f + p;   // the transpose view
-            const cbx_tensor* x = T(t, a.src[0]);
-            const cbx_tensor* al = pro == 1 ? T(t, a.src[1]) : nullptr;
-            const cbx_tensor* ai = pro == 1 ? T(t, nd[f + 3].src[1]) : nullptr;
-            const float slope = pro == 2 ? a.fparam : 0.0f;
-            const int cp = pro == 1 ? CBX_CONV_PRO_SNAKE : pro == 2 ? CBX_CONV_PRO_LEAKY_RELU : CBX_CONV_PRO_NONE;
-            const int32_t bview = b0 + (tr ? 5 : 7);   // the bias view, when there is one
-            const cbx_tensor* bt = bias ? T(t, nd[bview].src[0]) : nullptr;
-            // the prepared weights must be the node's weight tensor's
-            const cbx_gnode& wn = nd[b0 + (tr ? 2 : 5)];
-            const cbx_tensor* wk = T(t, nd[b0 + 2].src[0]);
-            if (!wk || !conv1d_weights_match(wn.conv_w, tr ? wn.conv[0] : 0, wk->ne[0], tr ? wk->ne[2] : wk->ne[1],
-                                             tr ? wk->ne[1] : wk->ne[2])) {
-                return set_error(CBX_ERR_INVALID_ARG, "cbx_graph_launch: node " + std::to_string(b0 + (tr ? 2 : 5)) +
-                                                          ": conv_w was not made from the node's weight tensor");
-            }
-            if (!tr) {
-                const cbx_gnode& ic = nd[b0 + 2];
-                const cbx_tensor* r = nullptr;
-                if (res) {
-                    const cbx_gnode& ra = nd[f + n_res - 1];   // add(residual, conv out)
-                    const int32_t out = nd[f + n_res - 2].dst;
-                    r = T(t, ra.src[0] == out ? ra.src[1] : ra.src[0]);
-                }
-                if (!sum) {
-                    return cbx_conv1d(x, nd[b0 + 5].conv_w, ic.conv[0], ic.conv[1], ic.conv[2], cp, al, ai, slope, bt,
-                                      r, y, s);
-                }
-                const cbx_gnode& sa = nd[f + n_res];          // add(acc, residual's result)
-                const int32_t rr = nd[f + n_res - 1].dst;
-                if (sa.op != CBX_GOP_ADD || (sa.src[0] != rr && sa.src[1] != rr)) break;
-                const cbx_tensor* acc = T(t, sa.src[0] == rr ? sa.src[1] : sa.src[0]);
-                float sc = 1.0f;
-                if (scl) {
-                    const cbx_gnode& sn = nd[f + n_res + 1];
-                    if (sn.op != CBX_GOP_SCALE || sn.src[0] != sa.dst) break;
-                    sc = sn.fparam;
-                }
-                return cbx_conv1d_sum(x, nd[b0 + 5].conv_w, ic.conv[0], ic.conv[1], ic.conv[2], cp, al, ai, slope, bt,
-                                      r, acc, sc, y, s);
-            }
-            // the crop: the view's offset into the full output, in frames
-            const cbx_tensor* full = T(t, nd[b0 + 2].dst);
-            const cbx_tensor* crop = T(t, nd[b0 + 3].dst);
-            if (!full || !crop) break;
-            const int64_t off = static_cast<const char*>(crop->data) - static_cast<const char*>(full->data);
-            if (off < 0 || off % 4 || off / 4 > (int64_t{1} << 30)) break;
-            return cbx_conv_transpose1d(x, nd[b0 + 2].conv_w, static_cast<int>(off / 4), cp, al, ai, slope, bt, y, s);
+            ConvCall c;
+            const int rc = conv_call_of(t, nd, l, &c);
+            if (rc == kConvMisfit) break;
+            if (rc) return rc;
+            if (l.kind == CBX_GL_CONV1D) return conv1d_call(c, s);
+            return cbx_conv_transpose1d(c.x, c.w, c.pad, c.prologue, c.alpha, c.alpha_inv, c.slope, c.bias, c.y, s);
         }
         case CBX_GL_CAUSAL_CONV1D: {
             // [mask ->] 12 nodes [+ bias 2]
@@ -1206,6 +1225,143 @@ int run(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const cbx_gla
             break;
     }
     return set_error(CBX_ERR_INVALID_ARG, "cbx_graph_launch: launch does not fit the node list");
+}
+
+// ---- what is issued for a plan ----------------------------------------------
+// A step of a recording or an eager run: one planned launch, or the launches
+// of up to kResMax ResBlock layers (two each: snake -> conv, snake -> conv ->
+// residual add) that one kernel runs (k_resblock.hip).  The plan says which
+// values are stored; a layer's conv1 output is the one planned store a step
+// leaves out, under the same terms as a chain's intermediates: nothing else
+// reads it and the caller does not keep it.
+struct Step {
+    int32_t n = 0;                    // planned launches: 1, or 2 per layer
+    int32_t li[2 * kResMax];
+    bool operator==(const Step& o) const { return n == o.n && std::equal(li, li + n, o.li); }
+};
+
+struct Scheduler {
+    const cbx_tensor* t;
+    const cbx_gnode* nd;
+    const std::vector<cbx_glaunch>& ls;
+    std::vector<int32_t> uses;
+    std::vector<char> keep;
+    struct Layer {
+        int ch = 0;
+        ConvCall c1, c2;
+    };
+    std::vector<Layer> layers;        // by step; ch 0: not a layer step
+
+    // planned launches i and i + 1 are a ResBlock layer
+    bool layer_at(size_t i, Layer* y) const {
+        if (i + 1 >= ls.size() || ls[i].kind != CBX_GL_CONV1D || ls[i + 1].kind != CBX_GL_CONV1D ||
+            (ls[i].flags & 3) != 1 || (ls[i + 1].flags & 3) != 1) {
+            return false;
+        }
+        const int32_t h = nd[ls[i].first_node + ls[i].n_nodes - 1].dst;
+        // snake reads its input twice: mul(x, alpha) and add(x, .)
+        if (keep[static_cast<size_t>(h)] || uses[static_cast<size_t>(h)] != 2 || nd[ls[i + 1].first_node].src[0] != h ||
+            nd[ls[i + 1].first_node + 4].src[0] != h) {
+            return false;
+        }
+        ResLayer r;
+        return conv_call_of(t, nd, ls[i], &y->c1) == CBX_OK && conv_call_of(t, nd, ls[i + 1], &y->c2) == CBX_OK &&
+               res_layer_of(y->c1, y->c2, &r, &y->ch);
+    }
+
+    // the layer (its reads and its one store) meets no store of planned
+    // launch l and l reads none of its output, by bytes; l's unstored
+    // intermediates count as stored
+    static bool apart(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, const Layer& y) {
+        for (int32_t i = l.first_node; i < l.first_node + l.n_nodes; i++) {
+            const cbx_tensor* d = &t[nd[i].dst];
+            for (const cbx_tensor* r : {y.c1.x, y.c1.alpha, y.c1.alpha_inv, y.c1.bias, y.c2.alpha, y.c2.alpha_inv,
+                                        y.c2.bias, y.c2.res, y.c2.acc, static_cast<const cbx_tensor*>(y.c2.y)}) {
+                if (r && bytes_overlap(d, r)) return false;
+            }
+            for (int32_t s : nd[i].src) {
+                if (s >= 0 && bytes_overlap(&t[s], y.c2.y)) return false;
+            }
+        }
+        return true;
+    }
+
+    std::vector<Step> run() {
+        std::vector<Step> steps;
+        for (size_t i = 0; i < ls.size();) {
+            Step s;
+            Layer y;
+            s.li[s.n++] = static_cast<int32_t>(i);
+            if (layer_at(i, &y)) s.li[s.n++] = static_cast<int32_t>(i + 1);
+            else y.ch = 0;
+            i += static_cast<size_t>(s.n);
+            steps.push_back(s);
+            layers.push_back(y);
+        }
+        // A layer joins an earlier one of its channel count when every step
+        // between them (and the layers already in that step) is independent
+        // of it: a stage's three ResBlocks read the same input and meet only
+        // in the sums of their last layers.
+        for (size_t i = 0; i < steps.size(); i++) {
+            if (!layers[i].ch) continue;
+            for (size_t j = i + 1; j < steps.size() && steps[i].n < 2 * kResMax;) {
+                bool ok = layers[j].ch == layers[i].ch && steps[j].n == 2;
+                for (size_t q = i; ok && q < j; q++) {
+                    for (int32_t m = 0; ok && m < steps[q].n; m++) {
+                        ok = apart(t, nd, ls[static_cast<size_t>(steps[q].li[m])], layers[j]);
+                    }
+                }
+                if (!ok) {
+                    j++;
+                    continue;
+                }
+                for (int32_t m = 0; m < 2; m++) steps[i].li[steps[i].n++] = steps[j].li[m];
+                steps.erase(steps.begin() + static_cast<std::ptrdiff_t>(j));
+                layers.erase(layers.begin() + static_cast<std::ptrdiff_t>(j));
+            }
+        }
+        return steps;
+    }
+};
+
+std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd, int32_t n,
+                           const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep) {
+    Scheduler s{t, nd, ls, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
+                std::vector<char>(static_cast<size_t>(n_t), 0), {}};
+    for (int32_t k = 0; k < n_keep; k++) s.keep[static_cast<size_t>(keep[k])] = 1;
+    for (int32_t i = 0; i < n; i++) {
+        for (int32_t q : nd[i].src) {
+            if (q >= 0) s.uses[static_cast<size_t>(q)]++;
+        }
+    }
+    return s.run();
+}
+
+// Issues a step.  *at names the planned launch an error belongs to.
+int run_step(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const std::vector<cbx_glaunch>& ls,
+             const Step& st, cbx_stream s, int32_t* at) {
+    *at = st.li[0];
+    if (st.n == 1) return run(t, nd, n_nodes, ls[static_cast<size_t>(st.li[0])], s);
+    int rc = CBX_OK;
+    DeviceState* ds = current_state(&rc);
+    if (!ds) return rc;
+    ResLayer r[kResMax];
+    int ch = 0;
+    for (int32_t m = 0; m < st.n; m += 2) {
+        ConvCall c1, c2;
+        if (conv_call_of(t, nd, ls[static_cast<size_t>(st.li[m])], &c1) ||
+            conv_call_of(t, nd, ls[static_cast<size_t>(st.li[m + 1])], &c2) || !res_layer_of(c1, c2, &r[m / 2], &ch)) {
+            return set_error(CBX_ERR_INVALID_ARG, "a ResBlock layer changed under its schedule");
+        }
+    }
+    return launch_res_layers(r, st.n / 2, ch, ds, reinterpret_cast<hipStream_t>(s));
+}
+
+// The planned launches of a step that run something (views do not)
+int32_t step_launches(const std::vector<cbx_glaunch>& ls, const Step& st) {
+    int32_t n = 0;
+    for (int32_t m = 0; m < st.n; m++) n += ls[static_cast<size_t>(st.li[m])].kind != CBX_GL_VIEW;
+    return n;
 }
 
 }  // namespace
@@ -1250,23 +1406,24 @@ int cbx_graph_launch(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gno
 // stream the exec was launched on since the one before, mark them (one
 // event a stream per update, none per replay).
 //
-// Each instantiation remembers the plan it holds, each launch's signature
-// (every value its kernels are built from) and which of its graph's kernel
-// nodes each launch issued.  An update whose plan has the same launches
-// re-records only the launches whose signature changed and sets their
+// Each instantiation remembers the plan and the steps it holds, each step's
+// signature (every value its kernels are built from) and which of its graph's
+// kernel nodes each step issued.  An update whose plan has the same launches
+// and steps re-records only the steps whose signature changed and sets their
 // kernel nodes' arguments in the instantiated graph (a decode loop's next
 // token changes a few launches of many); anything else records the whole
 // list and updates or re-instantiates the graph.
 struct GraphInst {
     hipGraph_t graph = nullptr;            // the graph `exec` was instantiated from
     hipGraphExec_t exec = nullptr;
-    int32_t n_launches = 0;                // kernel launches of one replay
+    int32_t n_launches = 0;                // planned launches of one replay
     bool indexed = false;                  // the fields below describe `exec`
     std::vector<hipGraphNode_t> knodes;    // graph's kernel nodes in launch order
     std::vector<cbx_glaunch> ls;           // the plan it holds
-    std::vector<int32_t> k0, kn;           // per launch: first kernel node, kernel count
-    std::vector<uint64_t> sig;             // the launches' signatures, back to back
-    std::vector<size_t> sig_at;            // launch i's signature: [sig_at[i], sig_at[i + 1])
+    std::vector<Step> steps;               // what it issues for it
+    std::vector<int32_t> k0, kn;           // per step: first kernel node, kernel count
+    std::vector<uint64_t> sig;             // the steps' signatures, back to back
+    std::vector<size_t> sig_at;            // step i's signature: [sig_at[i], sig_at[i + 1])
 };
 
 struct cbx_graph_exec {
@@ -1342,11 +1499,11 @@ static void launch_signature(const cbx_tensor* t, const cbx_gnode* nd, const cbx
 }
 
 static void signatures(const cbx_tensor* t, const cbx_gnode* nd, const std::vector<cbx_glaunch>& ls,
-                       std::vector<uint64_t>* sig, std::vector<size_t>* at) {
+                       const std::vector<Step>& steps, std::vector<uint64_t>* sig, std::vector<size_t>* at) {
     sig->clear();
     at->assign(1, 0);
-    for (const cbx_glaunch& l : ls) {
-        launch_signature(t, nd, l, sig);
+    for (const Step& st : steps) {
+        for (int32_t m = 0; m < st.n; m++) launch_signature(t, nd, ls[static_cast<size_t>(st.li[m])], sig);
         at->push_back(sig->size());
     }
 }
@@ -1388,15 +1545,16 @@ static int refuse_unsupported(const cbx_gnode* nodes, const std::vector<cbx_glau
     return CBX_OK;
 }
 
-// Records launches ls[which[0]], ls[which[1]], .. (every launch when which
-// is NULL) on cs (a stream of the exec's own, so nothing else the caller has
+// Records steps[which[0]], steps[which[1]], .. (every step when which is
+// NULL) on cs (a stream of the exec's own, so nothing else the caller has
 // queued ends up in the graph) into a new HIP graph (*out); kcount[j] gets
-// the kernel nodes launch j of the recording added (-1 when that could not
-// be read) and *issued the kernel launch count.  f names the caller in
+// the kernel nodes step j of the recording added (-1 when that could not be
+// read) and *issued the count of planned launches.  f names the caller in
 // errors.
 static int record(const cbx_tensor* tensors, const cbx_gnode* nodes, int32_t n_nodes,
-                  const std::vector<cbx_glaunch>& ls, const std::vector<int32_t>* which, hipStream_t cs,
-                  hipGraph_t* out, std::vector<int32_t>* kcount, int32_t* issued, const char* f) {
+                  const std::vector<cbx_glaunch>& ls, const std::vector<Step>& steps,
+                  const std::vector<int32_t>* which, hipStream_t cs, hipGraph_t* out, std::vector<int32_t>* kcount,
+                  int32_t* issued, const char* f) {
     *out = nullptr;
     *issued = 0;
     kcount->clear();
@@ -1407,17 +1565,19 @@ static int record(const cbx_tensor* tensors, const cbx_gnode* nodes, int32_t n_n
     int32_t n = 0;
     size_t before = 0;
     std::string inner;
-    const size_t count = which ? which->size() : ls.size();
+    const size_t count = which ? which->size() : steps.size();
     for (size_t j = 0; j < count; j++) {
-        const cbx_glaunch& l = ls[which ? static_cast<size_t>((*which)[j]) : j];
-        rc = run(tensors, nodes, n_nodes, l, cs);
+        const Step& st = steps[which ? static_cast<size_t>((*which)[j]) : j];
+        int32_t at = 0;
+        rc = run_step(tensors, nodes, n_nodes, ls, st, cs, &at);
         if (rc) {
+            const cbx_glaunch& l = ls[static_cast<size_t>(at)];
             inner = "nodes " + std::to_string(l.first_node) + ".." + std::to_string(l.first_node + l.n_nodes - 1) +
                     ": " + cbx_last_error();
             break;
         }
-        if (l.kind != CBX_GL_VIEW) n++;
-        // the nodes the capture holds now, less those before this launch
+        n += step_launches(ls, st);
+        // the nodes the capture holds now, less those before this step
         hipStreamCaptureStatus cst;
         hipGraph_t cg = nullptr;
         size_t now = 0;
@@ -1442,17 +1602,19 @@ static int record(const cbx_tensor* tensors, const cbx_gnode* nodes, int32_t n_n
 }
 
 // Fills an instantiation's bookkeeping for the plan it now holds, recorded
-// with per-launch kernel counts kcount; indexed stays false when the
-// graph's kernel nodes cannot be matched to the launches.
+// with per-step kernel counts kcount; indexed stays false when the graph's
+// kernel nodes cannot be matched to the steps.
 static void index_inst(GraphInst* t, const cbx_tensor* tensors, const cbx_gnode* nodes,
-                       const std::vector<cbx_glaunch>& ls, const std::vector<int32_t>& kcount, bool keep_nodes) {
+                       const std::vector<cbx_glaunch>& ls, const std::vector<Step>& steps,
+                       const std::vector<int32_t>& kcount, bool keep_nodes) {
     t->indexed = false;
     t->ls = ls;
-    signatures(tensors, nodes, ls, &t->sig, &t->sig_at);
-    t->k0.assign(ls.size(), 0);
-    t->kn.assign(ls.size(), 0);
+    t->steps = steps;
+    signatures(tensors, nodes, ls, steps, &t->sig, &t->sig_at);
+    t->k0.assign(steps.size(), 0);
+    t->kn.assign(steps.size(), 0);
     int32_t at = 0;
-    for (size_t i = 0; i < ls.size(); i++) {
+    for (size_t i = 0; i < steps.size(); i++) {
         if (i >= kcount.size() || kcount[i] < 0) return;
         t->k0[i] = at;
         t->kn[i] = kcount[i];
@@ -1476,6 +1638,7 @@ int cbx_graph_exec_create(const cbx_tensor* tensors, int32_t n_tensors, const cb
         (rc = refuse_unsupported(nodes, ls, f))) {
         return rc;
     }
+    const std::vector<Step> steps = schedule(tensors, n_tensors, nodes, n_nodes, ls, keep, n_keep);
     hipStream_t cs = nullptr;
     if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) {
         return set_error(CBX_ERR_HIP, std::string(f) + ": stream creation failed");
@@ -1483,7 +1646,7 @@ int cbx_graph_exec_create(const cbx_tensor* tensors, int32_t n_tensors, const cb
     hipGraph_t g[2] = {nullptr, nullptr};
     int32_t issued = 0;
     std::vector<int32_t> kcount;
-    rc = record(tensors, nodes, n_nodes, ls, nullptr, cs, &g[0], &kcount, &issued, f);
+    rc = record(tensors, nodes, n_nodes, ls, steps, nullptr, cs, &g[0], &kcount, &issued, f);
     if (rc == CBX_OK && hipGraphClone(&g[1], g[0]) != hipSuccess) {
         rc = set_error(CBX_ERR_HIP, std::string(f) + ": graph clone failed");
     }
@@ -1510,7 +1673,7 @@ int cbx_graph_exec_create(const cbx_tensor* tensors, int32_t n_tensors, const cb
         t.graph = g[k];
         t.exec = ge[k];
         t.n_launches = issued;
-        index_inst(&t, tensors, nodes, ls, kcount, false);
+        index_inst(&t, tensors, nodes, ls, steps, kcount, false);
     }
     x->cur = 0;
     *out = x;
@@ -1518,15 +1681,16 @@ int cbx_graph_exec_create(const cbx_tensor* tensors, int32_t n_tensors, const cb
     return CBX_OK;
 }
 
-// The targeted update: the launches whose signature changed, recorded
+// The targeted update: the steps whose signature changed, recorded
 // alone, their kernels' arguments set on t's kernel nodes.  *done = false
 // (and nothing fatal) when the update has to take the whole-list path.
 static int update_changed(cbx_graph_exec* x, GraphInst& t, const cbx_tensor* tensors, const cbx_gnode* nodes,
-                          int32_t n_nodes, const std::vector<cbx_glaunch>& ls, const std::vector<uint64_t>& sig,
-                          const std::vector<size_t>& sig_at, bool* done, const char* f) {
+                          int32_t n_nodes, const std::vector<cbx_glaunch>& ls, const std::vector<Step>& steps,
+                          const std::vector<uint64_t>& sig, const std::vector<size_t>& sig_at, bool* done,
+                          const char* f) {
     *done = false;
     std::vector<int32_t> changed;
-    for (size_t i = 0; i < ls.size(); i++) {
+    for (size_t i = 0; i < steps.size(); i++) {
         const size_t a = sig_at[i], b = sig_at[i + 1];
         if (b - a != t.sig_at[i + 1] - t.sig_at[i] ||
             !std::equal(sig.begin() + static_cast<std::ptrdiff_t>(a), sig.begin() + static_cast<std::ptrdiff_t>(b),
@@ -1538,7 +1702,7 @@ static int update_changed(cbx_graph_exec* x, GraphInst& t, const cbx_tensor* ten
         hipGraph_t g = nullptr;
         std::vector<int32_t> kcount;
         int32_t issued = 0;
-        int rc = record(tensors, nodes, n_nodes, ls, &changed, x->cs, &g, &kcount, &issued, f);
+        int rc = record(tensors, nodes, n_nodes, ls, steps, &changed, x->cs, &g, &kcount, &issued, f);
         if (rc) return rc;   // t untouched
         std::vector<hipGraphNode_t> gn;
         bool ok = kernel_chain(g, &gn);
@@ -1548,7 +1712,7 @@ static int update_changed(cbx_graph_exec* x, GraphInst& t, const cbx_tensor* ten
             want += static_cast<size_t>(kcount[j] > 0 ? kcount[j] : 0);
         }
         ok = ok && gn.size() == want;
-        // each changed launch's kernels, in order, onto the nodes it issued
+        // each changed step's kernels, in order, onto the nodes it issued
         size_t p = 0;
         for (size_t j = 0; ok && j < changed.size(); j++) {
             const size_t i = static_cast<size_t>(changed[j]);
@@ -1595,8 +1759,9 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
         (rc = refuse_unsupported(nodes, ls, f))) {
         return rc;   // exec is left as it was
     }
+    const std::vector<Step> steps = schedule(tensors, n_tensors, nodes, n_nodes, ls, keep, n_keep);
     GraphInst& t = exec->inst[1 - exec->cur];
-    bool same_plan = t.indexed && ls.size() == t.ls.size();
+    bool same_plan = t.indexed && ls.size() == t.ls.size() && steps == t.steps;
     for (size_t i = 0; same_plan && i < ls.size(); i++) {
         same_plan = ls[i].kind == t.ls[i].kind && ls[i].first_node == t.ls[i].first_node &&
                     ls[i].n_nodes == t.ls[i].n_nodes && ls[i].flags == t.ls[i].flags;
@@ -1604,13 +1769,13 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
     if (same_plan) {
         std::vector<uint64_t> sig;
         std::vector<size_t> sig_at;
-        signatures(tensors, nodes, ls, &sig, &sig_at);
+        signatures(tensors, nodes, ls, steps, &sig, &sig_at);
         // the instantiation to re-point is the one not replayed since the
         // last update: wait for its replays (issued before that update),
         // then mark the current one's
         if ((rc = wait_marks(exec, f)) || (rc = mark_launches(exec, f))) return rc;
         bool done = false;
-        if ((rc = update_changed(exec, t, tensors, nodes, n_nodes, ls, sig, sig_at, &done, f))) return rc;
+        if ((rc = update_changed(exec, t, tensors, nodes, n_nodes, ls, steps, sig, sig_at, &done, f))) return rc;
         if (done) {
             exec->cur = 1 - exec->cur;
             if (n_launches) *n_launches = t.n_launches;
@@ -1621,7 +1786,7 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
     hipGraph_t g = nullptr;
     int32_t issued = 0;
     std::vector<int32_t> kcount;
-    rc = record(tensors, nodes, n_nodes, ls, nullptr, exec->cs, &g, &kcount, &issued, f);
+    rc = record(tensors, nodes, n_nodes, ls, steps, nullptr, exec->cs, &g, &kcount, &issued, f);
     if (rc) return rc;   // exec is left as it was
     if (!same_plan && ((rc = wait_marks(exec, f)) || (rc = mark_launches(exec, f)))) {
         (void)hipGraphDestroy(g);
@@ -1634,7 +1799,7 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
     if (issued == t.n_launches && hipGraphExecUpdate(t.exec, g, &bad_node, &res) == hipSuccess &&
         res == hipGraphExecUpdateSuccess) {
         (void)hipGraphDestroy(g);
-        index_inst(&t, tensors, nodes, ls, kcount, true);
+        index_inst(&t, tensors, nodes, ls, steps, kcount, true);
         exec->cur = 1 - exec->cur;
         if (n_launches) *n_launches = issued;
         if (in_place) *in_place = 1;
@@ -1652,7 +1817,7 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
     t.graph = g;
     t.exec = ge;
     t.n_launches = issued;
-    index_inst(&t, tensors, nodes, ls, kcount, false);
+    index_inst(&t, tensors, nodes, ls, steps, kcount, false);
     exec->cur = 1 - exec->cur;
     if (n_launches) *n_launches = issued;
     return CBX_OK;
@@ -1714,14 +1879,16 @@ int cbx_graph_compute(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gn
         }
     }
     int32_t issued = 0;
-    for (const cbx_glaunch& l : ls) {
-        rc = run(tensors, nodes, n_nodes, l, stream);
+    for (const Step& st : schedule(tensors, n_tensors, nodes, n_nodes, ls, keep, n_keep)) {
+        int32_t at = 0;
+        rc = run_step(tensors, nodes, n_nodes, ls, st, stream, &at);
         if (rc) {
+            const cbx_glaunch& l = ls[static_cast<size_t>(at)];
             const std::string inner = cbx_last_error();
             return set_error(rc, "cbx_graph_compute: nodes " + std::to_string(l.first_node) + ".." +
                                      std::to_string(l.first_node + l.n_nodes - 1) + ": " + inner);
         }
-        if (l.kind != CBX_GL_VIEW) issued++;
+        issued += step_launches(ls, st);
         if (n_launches) *n_launches = issued;
     }
     return CBX_OK;

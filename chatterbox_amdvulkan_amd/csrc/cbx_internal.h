@@ -160,6 +160,41 @@ int launch_conv1d(const cbx_tensor* x, const _Float16* w16, int64_t k, int64_t c
                   int pad, int dil, int up, int crop, int64_t w_ph, int pro, const cbx_tensor* alpha,
                   const cbx_tensor* alpha_inv, float slope, const cbx_tensor* bias, const cbx_tensor* res, cbx_tensor* y,
                   DeviceState* st, hipStream_t s, const cbx_tensor* acc = nullptr, float oscale = 1.0f);
+// One ResBlock layer run by k_resblock.hip: y = res + conv2(snake2(conv1(
+// snake1(x)) + b1)) + b2, then [+ acc [* oscale]], all (ch, T) f32 with
+// 16-byte aligned rows at the given byte steps; both convs stride 1 with
+// "same" padding ((k - 1) * d even), w1 and w2 prepared weights.
+struct ResLayer {
+    const char* x;
+    const _Float16 *w1, *w2;
+    const float *al1, *ai1, *b1, *al2, *ai2, *b2;
+    const char *res, *acc;      // acc may be null
+    char* y;
+    int64_t x_nb1, r_nb1, a_nb1, y_nb1;
+    int32_t T, k1, d1, k2, d2;
+    int32_t scaled;             // the sum times oscale
+    float oscale;
+    int32_t tiles;              // set by the launcher
+};
+constexpr int kResMax = 3;      // layers of one launch
+// Whether the one-launch form takes the layer (and is the faster one).
+bool res_layer_fits(const ResLayer& l, int ch, const DeviceState* st);
+int launch_res_layers(const ResLayer* ls, int n, int ch, DeviceState* st, hipStream_t s);
+// The arguments of a cbx_conv1d (acc null) or cbx_conv1d_sum call.
+struct ConvCall {
+    const cbx_tensor* x;
+    const cbx_conv1d_weights* w;
+    int stride, pad, dilation, prologue;
+    const cbx_tensor *alpha, *alpha_inv;
+    float slope;
+    const cbx_tensor *bias, *res, *acc;
+    float scale;
+    cbx_tensor* y;
+};
+int conv1d_call(const ConvCall& c, cbx_stream stream);
+// Whether c1 then c2 are a ResBlock layer (c2 reads c1's output, which the
+// caller says nothing else reads) that one launch takes: *l is filled.
+bool res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int* ch);
 // Whether prepared weights were made from a weight of these extents: a
 // conv1d weight (K, C_in, C_out) when up == 0, else a transposed weight
 // (K, C_out, C_in) split for stride up.

@@ -39,6 +39,7 @@ SOURCES = [
     "k_resblock.hip",
     "k_eltwise.hip",
     "k_batch.hip",
+    "k_group.hip",
     "k_binary.hip",
 ]
 HEADERS = ["cbx_internal.h", "cbx_device.h", "cbx_rowops.h", os.path.join("..", "..", "include", "cbxops.h")]

@@ -1228,32 +1228,409 @@ int run(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const cbx_gla
 }
 
 // ---- what is issued for a plan ----------------------------------------------
-// A step of a recording or an eager run: one planned launch, or the launches
-// of up to kResMax ResBlock layers (two each: snake -> conv, snake -> conv ->
-// residual add) that one kernel runs (k_resblock.hip).  The plan says which
-// values are stored; a layer's conv1 output is the one planned store a step
-// leaves out, under the same terms as a chain's intermediates: nothing else
-// reads it and the caller does not keep it.
+// A plan's launches are issued as steps, each one kernel where it holds
+// several: the layers of independent ResBlocks (two launches each,
+// k_resblock.hip), element-wise launches or softmaxes that do not depend on
+// each other, and chains of dependent row launches (k_group.hip).  A launch
+// joins the earliest step of its kind that follows every step it conflicts
+// with, by the bytes it reads and stores, so the values are those of the
+// launches in their order.  A ResBlock layer's conv1 output is the one
+// planned store a step leaves out, under the terms of a chain's
+// intermediates: nothing else reads it and the caller does not keep it.
+enum { kStepOne = 0, kStepLayers, kStepElt, kStepSoftMax, kStepRows };
+constexpr int kStepMax = 48;
+static_assert(kStepMax <= kEltMax && kStepMax <= kSoftMaxGroup && kStepMax <= kChainMax && 2 * kResMax <= kStepMax, "");
+
 struct Step {
-    int32_t n = 0;                    // planned launches: 1, or 2 per layer
-    int32_t li[2 * kResMax];
-    bool operator==(const Step& o) const { return n == o.n && std::equal(li, li + n, o.li); }
+    int32_t kind = kStepOne;
+    int32_t n = 0;                    // planned launches (two per layer)
+    int32_t li[kStepMax];
+    bool operator==(const Step& o) const { return kind == o.kind && n == o.n && std::equal(li, li + n, o.li); }
 };
+
+bool f32_flat16(const cbx_tensor* t) {
+    return t && t->data && t->type == CBX_TYPE_F32 && is_contiguous(t) && reinterpret_cast<uintptr_t>(t->data) % 16 == 0;
+}
+
+// t is one row of n floats
+bool row_of(const cbx_tensor* t, int64_t n) { return f32_flat16(t) && t->ne[0] == n && nelements(t) == n; }
+
+// y = x op b: how b runs against x for the element-wise group, false when
+// it takes no such form.  y may be x itself and meets no other operand.
+bool elt_binary(const cbx_tensor* x, const cbx_tensor* b, const cbx_tensor* y, EltOp* e) {
+    const bool rows4 = x->ne[0] % 4 == 0;
+    if (!f32_flat16(x) || !f32_flat16(y) || !same_shape(x, y) || nelements(x) < 4 || nelements(x) % 4 ||
+        nelements(x) >= (int64_t{1} << 32) || (x->data != y->data && bytes_overlap(x, y))) {
+        return false;
+    }
+    *e = EltOp{};
+    e->x = static_cast<const float*>(x->data);
+    e->y = static_cast<float*>(y->data);
+    e->n4 = static_cast<uint32_t>(nelements(x) / 4);
+    e->ne0_4 = static_cast<uint32_t>(x->ne[0] / 4);
+    e->act = CBX_UNARY_NONE;
+    if (!b) return true;
+    if (b->type != CBX_TYPE_F32 || !b->data || !is_contiguous(b) || bytes_overlap(b, y)) return false;
+    e->b = static_cast<const float*>(b->data);
+    if (rows4 && row_of(b, x->ne[0])) {
+        e->bmode = kEltVec;
+        e->C = static_cast<uint32_t>(x->ne[0]);
+    } else if (b->ne[0] == 1 && b->ne[1] == x->ne[1] && nelements(b) == b->ne[1]) {
+        e->bmode = rows4 ? kEltRow : kEltRowAny;
+        if (!rows4) e->ne0_4 = static_cast<uint32_t>(x->ne[0]);
+        e->C = static_cast<uint32_t>(b->ne[1]);
+    } else if (f32_flat16(b) && same_shape(b, x)) {
+        e->bmode = kEltFull;
+    } else {
+        return false;
+    }
+    return true;
+}
+
+// The element-wise ops (at most two) of a planned launch: the count, or 0.
+int elt_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, EltOp e[2]) {
+    const int32_t f = l.first_node;
+    const cbx_gnode &a = nd[f], &z = nd[f + l.n_nodes - 1];
+    const cbx_tensor* x = T(t, a.src[0]);
+    const cbx_tensor* y = T(t, z.dst);
+    if (!x || !y) return 0;
+    switch (l.kind) {
+        case CBX_GL_BIAS_ACT: {
+            const cbx_tensor* b = T(t, a.src[1]);
+            if (l.n_nodes == 3 || !b || !elt_binary(x, b, y, e) || e->bmode == kEltFull) return 0;
+            e->act = l.n_nodes == 1 ? CBX_UNARY_NONE : l.n_nodes == 4 ? CBX_UNARY_MISH : nd[f + 1].iparam;
+            return 1;
+        }
+        case CBX_GL_BIAS_ADD_TWO:
+            for (int k = 0; k < 2; k++) {
+                const cbx_gnode& g = nd[f + k];
+                const cbx_tensor *gx = T(t, g.src[0]), *gb = T(t, g.src[1]);
+                if (g.op != CBX_GOP_ADD || !gx || !gb || !elt_binary(gx, gb, T(t, g.dst), e + k) ||
+                    e[k].bmode == kEltFull) {
+                    return 0;
+                }
+            }
+            return 2;
+        case CBX_GL_BIAS_ADD_PAIR: {
+            // add(x, bias) -> heads view -> [views] add(view, u), add(view, v)
+            const cbx_gnode& v = nd[f + 1];
+            const cbx_tensor *b = T(t, a.src[1]), *V = T(t, v.dst);
+            if (v.op != CBX_GOP_VIEW || !b || !V || !row_of(b, x->ne[0])) return 0;
+            int n = 0;
+            for (int32_t k = f + 2; k < f + l.n_nodes; k++) {
+                const cbx_gnode& g = nd[k];
+                if (g.op == CBX_GOP_VIEW) continue;
+                const cbx_tensor *u = T(t, g.src[1]), *o = T(t, g.dst);
+                // u spans whole leading dims of the view: one period of it
+                if (n == 2 || g.op != CBX_GOP_ADD || g.src[0] != v.dst || !f32_flat16(u) || !f32_flat16(o) ||
+                    !same_shape(o, V) || nelements(o) != nelements(x) || lead_dims(*V, nelements(u)) < 0 ||
+                    u->ne[0] != V->ne[0] || nelements(u) % 4) {
+                    return 0;
+                }
+                int64_t p = 1;   // u's own dims are the view's leading ones
+                for (int q = 0; q < 4; q++) {
+                    if (p < nelements(u) ? u->ne[q] != V->ne[q] : u->ne[q] != 1) return 0;
+                    p *= u->ne[q];
+                }
+                cbx_tensor oy = *x;   // the output re-described with x's shape
+                oy.data = o->data;
+                if (bytes_overlap(o, u) || bytes_overlap(o, x) || !elt_binary(x, b, &oy, e + n)) return 0;
+                e[n].b2 = static_cast<const float*>(u->data);
+                e[n].C2 = static_cast<uint32_t>(nelements(u));
+                n++;
+            }
+            if (n != 2) return 0;
+            return n;
+        }
+        case CBX_GL_UNARY:
+            if ((l.n_nodes != 1 && l.n_nodes != 3) || !elt_binary(x, nullptr, y, e)) return 0;
+            e->act = l.n_nodes == 3 ? CBX_UNARY_MISH : a.iparam;
+            return 1;
+        case CBX_GL_LEAKY_RELU:
+            if (!elt_binary(x, nullptr, y, e)) return 0;
+            e->act = UNARY_LEAKY;
+            e->param = a.fparam;
+            return 1;
+        case CBX_GL_SCALE:
+            if (a.op != CBX_GOP_SCALE || !elt_binary(x, nullptr, y, e)) return 0;
+            e->act = kEltScale;
+            e->param = a.fparam;
+            return 1;
+        case CBX_GL_BINARY: {
+            const cbx_tensor* b = T(t, a.src[1]);
+            if (!b || !elt_binary(x, b, y, e)) return 0;
+            e->mul = l.flags == CBX_BINARY_MUL;
+            return 1;
+        }
+        default: return 0;
+    }
+}
+
+// The copies of concats along dim 0 at planned launches li[0 .. n), each
+// appending to the one before it (whose result only it reads): one per
+// source, into the last one's result.  The count (n + 1), or 0.
+constexpr int kConcatMax = 4;
+int concat_of(const cbx_tensor* t, const cbx_gnode* nd, const std::vector<cbx_glaunch>& ls, const int32_t* li, int32_t n,
+              EltOp* e) {
+    auto N = [&](int32_t m) -> const cbx_gnode& { return nd[ls[static_cast<size_t>(li[m])].first_node]; };
+    const cbx_tensor* y = T(t, N(n - 1).dst);
+    if (n < 1 || n > kConcatMax || !f32_flat16(y) || nelements(y) >= (int64_t{1} << 32)) return 0;
+    int64_t off = 0;
+    int k = 0;
+    for (int32_t m = 0; m < n; m++) {
+        const cbx_gnode& g = N(m);
+        if (g.op != CBX_GOP_CONCAT || g.iparam != 0 || (m > 0 && g.src[0] != N(m - 1).dst)) return 0;
+        for (int q = m ? 1 : 0; q < 2; q++) {
+            const cbx_tensor* x = T(t, g.src[q]);
+            if (!f32_flat16(x) || x->ne[0] % 4 || nelements(x) < 4 || bytes_overlap(x, y)) return 0;
+            for (int d = 1; d < 4; d++) {
+                if (x->ne[d] != y->ne[d]) return 0;
+            }
+            e[k] = EltOp{};
+            e[k].x = static_cast<const float*>(x->data);
+            e[k].y = static_cast<float*>(y->data) + off;
+            e[k].n4 = static_cast<uint32_t>(nelements(x) / 4);
+            e[k].ne0_4 = static_cast<uint32_t>(x->ne[0] / 4);
+            e[k].ld4 = static_cast<uint32_t>(y->ne[0] / 4);
+            e[k].act = CBX_UNARY_NONE;
+            off += x->ne[0];
+            k++;
+        }
+    }
+    return off == y->ne[0] ? k : 0;
+}
+
+// A planned softmax as a call (run()'s reading of it), its group key >= 0.
+bool softmax_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, const DeviceState* st, SoftMaxCall* c,
+                int64_t* key) {
+    if (l.kind != CBX_GL_SOFT_MAX) return false;
+    const int32_t f = l.first_node, z = f + l.n_nodes - 1;
+    const bool add = nd[f].op == CBX_GOP_ADD;
+    *c = SoftMaxCall{T(t, nd[f].src[0]), add ? T(t, nd[f].src[1]) : nullptr, 1.0f, -1,
+                     const_cast<cbx_tensor*>(&t[nd[z].dst])};
+    if (nd[z].op != CBX_GOP_SOFT_MAX) return false;
+    if (l.n_nodes == 1) c->scale = nd[f].fparam;
+    for (int32_t k = add ? f + 1 : f; k < z; k++) {
+        if (nd[k].op == CBX_GOP_SCALE) c->scale = nd[k].fparam;
+        else if (nd[k].op == CBX_GOP_DIAG_MASK_INF && nd[k].iparam >= 0) c->n_past = nd[k].iparam;
+        else return false;
+    }
+    for (const cbx_tensor* p : {c->x, add ? c->b : c->x, static_cast<const cbx_tensor*>(c->y)}) {
+        if (!p || !p->data || p->type != CBX_TYPE_F32 || p->nb[0] != sizeof(float) || !same_shape(p, c->x) ||
+            nelements(p) == 0) {
+            return false;
+        }
+    }
+    // y may be x itself (each row is read before it is written)
+    bool same = c->x->data == c->y->data;
+    for (int q = 1; q < 4; q++) same = same && c->x->nb[q] == c->y->nb[q];
+    if ((!same && bytes_overlap(c->x, c->y)) || (add && bytes_overlap(c->b, c->y))) return false;
+    *key = soft_max_group_key(*c, st);
+    return *key >= 0;
+}
+
+// The operands of a row link: a (one row of ne0 floats when a_vec), ab, r,
+// w, b, mask as RowLink; s is the sum (its tensor also when it is not
+// stored), y the result (null for a link without a norm).
+struct LinkT {
+    const cbx_tensor *a, *ab, *r, *w, *b, *mask;
+    cbx_tensor *s, *y;
+    float eps, scale;
+    bool mish, a_vec, norm, scaled, store_s;
+    int64_t ne0, nr;
+};
+
+bool link_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, LinkT* k) {
+    const int32_t f = l.first_node, z = f + l.n_nodes - 1;
+    auto M = [&](int32_t i) { return const_cast<cbx_tensor*>(T(t, i)); };
+    *k = LinkT{};
+    k->scale = 1.0f;
+    cbx_tensor* out = M(nd[z].dst);
+    int32_t ln = -1;   // the norm node
+    switch (l.kind) {
+        case CBX_GL_LAYER_NORM:
+        case CBX_GL_LAYER_NORM_MASK: {
+            const int32_t m = l.kind == CBX_GL_LAYER_NORM_MASK ? 1 : 0;
+            if (l.n_nodes - m != 3 && l.n_nodes - m != 6) return false;
+            ln = f;
+            k->a = T(t, nd[f].src[0]);
+            k->s = M(nd[f].src[0]);
+            if (l.n_nodes - m == 6) k->mish = true;
+            if (m && !(k->mask = T(t, nd[z].src[1]))) return false;
+            break;
+        }
+        case CBX_GL_ADD_LAYER_NORM: {
+            if (l.n_nodes != 4 && l.n_nodes != 5 && l.n_nodes != 7 && l.n_nodes != 8) return false;
+            const bool bias = l.n_nodes == 5 || l.n_nodes == 8;
+            const int32_t j = bias ? f + 1 : f;   // the last add
+            ln = j + 1;
+            k->a = T(t, nd[f].src[0]);
+            const cbx_tensor* a1 = T(t, nd[f].src[1]);
+            if (!k->a || !a1) return false;
+            if (bias) {
+                k->ab = a1;
+                k->r = T(t, nd[j].src[0] == nd[f].dst ? nd[j].src[1] : nd[j].src[0]);
+                if (!k->r) return false;
+            } else if (same_shape(k->a, a1)) {
+                k->r = a1;
+            } else {
+                k->ab = a1;
+            }
+            k->s = M(nd[j].dst);
+            k->store_s = (l.flags & 1) == 0;
+            if (l.n_nodes >= 7) k->mish = true;
+            break;
+        }
+        case CBX_GL_BIAS_RESIDUAL: {
+            const int32_t sum = l.n_nodes == 3 ? nd[f + 1].dst : nd[f].dst;
+            k->a = T(t, nd[f].src[0]);
+            k->ab = T(t, nd[f].src[1]);
+            k->r = T(t, nd[z].src[0] == sum ? nd[z].src[1] : nd[z].src[0]);
+            if (!k->a || !k->ab || !k->r) return false;
+            k->s = out;
+            k->store_s = true;
+            k->a_vec = !same_shape(k->a, k->r);
+            break;
+        }
+        case CBX_GL_SCALE:
+            if (nd[f].op != CBX_GOP_SCALE) return false;
+            k->a = T(t, nd[f].src[0]);
+            k->s = M(nd[f].src[0]);
+            k->scale = nd[f].fparam;
+            k->scaled = true;
+            break;
+        case CBX_GL_BINARY:   // rows times their mask values
+            if (l.flags != CBX_BINARY_MUL || nd[f].op != CBX_GOP_MUL) return false;
+            k->a = T(t, nd[f].src[0]);
+            k->s = M(nd[f].src[0]);
+            k->mask = T(t, nd[f].src[1]);
+            if (!k->mask) return false;
+            break;
+        default: return false;
+    }
+    if (!k->a || !out) return false;
+    if (k->mask && (k->mask->type != CBX_TYPE_F32 || !k->mask->data || !is_contiguous(k->mask) || k->mask->ne[0] != 1 ||
+                    k->mask->ne[1] != k->a->ne[1] || nelements(k->mask) != nrows(k->a))) {
+        return false;
+    }
+    if (ln >= 0) {
+        k->norm = true;
+        k->eps = nd[ln].fparam;
+        k->w = T(t, nd[ln + 1].src[1]);
+        k->b = T(t, nd[ln + 2].src[1]);
+        if (!(k->eps >= 0.0f) || !row_of(k->w, out->ne[0]) || !row_of(k->b, out->ne[0])) return false;
+    }
+    if (ln >= 0 || k->scaled || k->mask) k->y = out;
+    k->ne0 = out->ne[0];
+    k->nr = nrows(out);
+    if (k->ne0 % 4 || k->ne0 > 1024 || k->nr < 1 || k->nr >= (int64_t{1} << 31)) return false;
+    if (k->a_vec ? !row_of(k->a, k->ne0) : (!f32_flat16(k->a) || !same_shape(k->a, out))) return false;
+    if (k->ab && !row_of(k->ab, k->ne0)) return false;
+    for (const cbx_tensor* p : {k->r, static_cast<const cbx_tensor*>(out), static_cast<const cbx_tensor*>(k->store_s ? k->s : nullptr)}) {
+        if (p && (!f32_flat16(p) || !same_shape(p, out))) return false;
+    }
+    // a link's stores meet none of its operands and not each other
+    for (const cbx_tensor* w : {static_cast<const cbx_tensor*>(k->store_s ? k->s : nullptr), static_cast<const cbx_tensor*>(k->y)}) {
+        if (!w) continue;
+        for (const cbx_tensor* p : {k->a, k->ab, k->r, k->w, k->b, k->mask}) {
+            if (p && bytes_overlap(w, p)) return false;
+        }
+    }
+    return !(k->store_s && k->y && bytes_overlap(k->s, k->y));
+}
+
+struct Span {
+    uintptr_t lo, hi;
+};
+
+Span span_of(const cbx_tensor& t) {
+    if (nelements(&t) <= 0) return Span{0, 0};
+    uintptr_t hi = reinterpret_cast<uintptr_t>(t.data) + type_size(t.type);
+    if (t.type == CBX_TYPE_Q8_0) hi = reinterpret_cast<uintptr_t>(t.data) + static_cast<uintptr_t>(t.ne[0] / 32 * 34);
+    for (int k = t.type == CBX_TYPE_Q8_0 ? 1 : 0; k < 4; k++) hi += static_cast<uintptr_t>(t.ne[k] - 1) * t.nb[k];
+    return Span{reinterpret_cast<uintptr_t>(t.data), hi};
+}
 
 struct Scheduler {
     const cbx_tensor* t;
     const cbx_gnode* nd;
     const std::vector<cbx_glaunch>& ls;
+    const DeviceState* st;
     std::vector<int32_t> uses;
     std::vector<char> keep;
-    struct Layer {
-        int ch = 0;
-        ConvCall c1, c2;
-    };
-    std::vector<Layer> layers;        // by step; ch 0: not a layer step
 
-    // planned launches i and i + 1 are a ResBlock layer
-    bool layer_at(size_t i, Layer* y) const {
+    // What the next launch to join a step is matched on.
+    struct Info {
+        int64_t key = 0;                        // layers: channels; softmax: its key
+        LinkT link;                             // rows: the last link
+        int elts = 0;                           // element-wise ops
+    };
+    std::vector<Step> steps;
+    std::vector<Info> info;
+    // Tensors whose bytes meet, directly or through others, are one class;
+    // the last step that reads and that writes a class is all a launch has
+    // to look at.
+    std::vector<int32_t> cls;                   // by tensor; -1: no bytes
+    std::vector<int32_t> last_rd, last_wr;      // by class: the last step, or -1
+    std::vector<int32_t> rd, wr;                // the current launch's classes
+
+    void classes(int32_t n_t) {
+        std::vector<std::pair<Span, int32_t>> v;
+        v.reserve(static_cast<size_t>(n_t));
+        cls.assign(static_cast<size_t>(n_t), -1);
+        for (int32_t i = 0; i < n_t; i++) {
+            const Span p = span_of(t[i]);
+            if (p.hi > p.lo) v.push_back({p, i});
+        }
+        std::sort(v.begin(), v.end(), [](const auto& x, const auto& y) { return x.first.lo < y.first.lo; });
+        int32_t n = -1;
+        uintptr_t hi = 0;
+        for (const auto& q : v) {
+            if (n < 0 || q.first.lo >= hi) {
+                n++;
+                hi = 0;
+            }
+            hi = std::max(hi, q.first.hi);
+            cls[static_cast<size_t>(q.second)] = n;
+        }
+        last_rd.assign(static_cast<size_t>(n + 1), -1);
+        last_wr.assign(static_cast<size_t>(n + 1), -1);
+    }
+
+    void touch(std::vector<int32_t>* v, int32_t tensor) {
+        const int32_t c = cls[static_cast<size_t>(tensor)];
+        if (c >= 0) v->push_back(c);
+    }
+
+    // Adds what a launch reads and stores to rd and wr: its nodes' operands
+    // and results, less the intermediates that only its own nodes read and
+    // nothing keeps (never stored).  A view stands for its source.
+    void accesses(const cbx_glaunch& l) {
+        const int32_t a = l.first_node, z = l.first_node + l.n_nodes;
+        for (int32_t i = a; i < z; i++) {
+            if (nd[i].op != CBX_GOP_VIEW && !inner(l, nd[i].dst, i)) touch(&wr, nd[i].dst);
+            for (int32_t s : nd[i].src) {
+                if (s < 0) continue;
+                bool made = false;   // by a node of the launch
+                for (int32_t j = a; j < i; j++) made = made || nd[j].dst == s;
+                if (!made) touch(&rd, s);
+            }
+        }
+    }
+
+    // tensor d, made by node i of launch l, stays unstored: a later node of
+    // the launch reads it, nothing outside does, and it is not kept
+    bool inner(const cbx_glaunch& l, int32_t d, int32_t i) const {
+        if (keep[static_cast<size_t>(d)] || i + 1 == l.first_node + l.n_nodes) return false;
+        int32_t in = 0;
+        for (int32_t j = i + 1; j < l.first_node + l.n_nodes; j++) {
+            for (int32_t s : nd[j].src) in += s == d;
+        }
+        return in > 0 && in == uses[static_cast<size_t>(d)];
+    }
+
+    // planned launches i and i + 1 are a ResBlock layer of *ch channels
+    bool layer_at(size_t i, int* ch) const {
         if (i + 1 >= ls.size() || ls[i].kind != CBX_GL_CONV1D || ls[i + 1].kind != CBX_GL_CONV1D ||
             (ls[i].flags & 3) != 1 || (ls[i + 1].flags & 3) != 1) {
             return false;
@@ -1265,60 +1642,130 @@ struct Scheduler {
             return false;
         }
         ResLayer r;
-        return conv_call_of(t, nd, ls[i], &y->c1) == CBX_OK && conv_call_of(t, nd, ls[i + 1], &y->c2) == CBX_OK &&
-               res_layer_of(y->c1, y->c2, &r, &y->ch);
+        ConvCall c1, c2;
+        const bool ok = conv_call_of(t, nd, ls[i], &c1) == CBX_OK && conv_call_of(t, nd, ls[i + 1], &c2) == CBX_OK &&
+                        res_layer_of(c1, c2, &r, ch);
+        clear_error();
+        return ok;
     }
 
-    // the layer (its reads and its one store) meets no store of planned
-    // launch l and l reads none of its output, by bytes; l's unstored
-    // intermediates count as stored
-    static bool apart(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, const Layer& y) {
-        for (int32_t i = l.first_node; i < l.first_node + l.n_nodes; i++) {
-            const cbx_tensor* d = &t[nd[i].dst];
-            for (const cbx_tensor* r : {y.c1.x, y.c1.alpha, y.c1.alpha_inv, y.c1.bias, y.c2.alpha, y.c2.alpha_inv,
-                                        y.c2.bias, y.c2.res, y.c2.acc, static_cast<const cbx_tensor*>(y.c2.y)}) {
-                if (r && bytes_overlap(d, r)) return false;
-            }
-            for (int32_t s : nd[i].src) {
-                if (s >= 0 && bytes_overlap(&t[s], y.c2.y)) return false;
-            }
+    // Link k may follow the chain that is step `at`: the rows match, what it
+    // reads of the chain's stores is exactly the last link's sum or result
+    // (which it takes from registers), and its stores meet nothing the chain
+    // reads or stores.
+    bool follows(size_t at, const LinkT& k) const {
+        const LinkT& p = info[at].link;
+        const int32_t me = static_cast<int32_t>(at);
+        if (p.ne0 != k.ne0 || p.nr != k.nr) return false;
+        for (const cbx_tensor* q : {k.a, k.ab, k.r, k.w, k.b, k.mask}) {
+            if (!q) continue;
+            const bool reg = (q == k.a && !k.a_vec) || q == k.r;
+            if (reg && from_chain(p, q) != kFromMemory) continue;
+            const int32_t c = cls[static_cast<size_t>(q - t)];
+            if (c >= 0 && last_wr[static_cast<size_t>(c)] == me) return false;
+        }
+        for (const cbx_tensor* q : {static_cast<const cbx_tensor*>(k.store_s ? k.s : nullptr), static_cast<const cbx_tensor*>(k.y)}) {
+            const int32_t c = q ? cls[static_cast<size_t>(q - t)] : -1;
+            if (c >= 0 && (last_wr[static_cast<size_t>(c)] == me || last_rd[static_cast<size_t>(c)] == me)) return false;
         }
         return true;
     }
 
-    std::vector<Step> run() {
-        std::vector<Step> steps;
+    // where a link after p finds operand q
+    static uint32_t from_chain(const LinkT& p, const cbx_tensor* q) {
+        if (p.y && q->data == p.y->data) return kFromResult;
+        if (p.s && (p.store_s || p.s == p.a) && q->data == p.s->data) return p.y ? kFromSum : kFromResult;
+        return kFromMemory;
+    }
+
+    // planned launch i appends (a concat along dim 0) to launch i - 1's
+    // result, which nothing else reads and nothing keeps
+    bool appends(size_t i) const {
+        if (i >= ls.size() || ls[i].kind != CBX_GL_CONCAT || ls[i - 1].kind != CBX_GL_CONCAT) return false;
+        const int32_t d = nd[ls[i - 1].first_node].dst;
+        return nd[ls[i].first_node].src[0] == d && nd[ls[i].first_node].src[1] != d &&
+               uses[static_cast<size_t>(d)] == 1 && !keep[static_cast<size_t>(d)];
+    }
+
+    std::vector<Step>& run(int32_t n_t) {
+        classes(n_t);
         for (size_t i = 0; i < ls.size();) {
+            const cbx_glaunch& l = ls[i];
+            const size_t at = i++;
+            if (l.kind == CBX_GL_VIEW) continue;
+            Info f;
             Step s;
-            Layer y;
-            s.li[s.n++] = static_cast<int32_t>(i);
-            if (layer_at(i, &y)) s.li[s.n++] = static_cast<int32_t>(i + 1);
-            else y.ch = 0;
-            i += static_cast<size_t>(s.n);
-            steps.push_back(s);
-            layers.push_back(y);
-        }
-        // A layer joins an earlier one of its channel count when every step
-        // between them (and the layers already in that step) is independent
-        // of it: a stage's three ResBlocks read the same input and meet only
-        // in the sums of their last layers.
-        for (size_t i = 0; i < steps.size(); i++) {
-            if (!layers[i].ch) continue;
-            for (size_t j = i + 1; j < steps.size() && steps[i].n < 2 * kResMax;) {
-                bool ok = layers[j].ch == layers[i].ch && steps[j].n == 2;
-                for (size_t q = i; ok && q < j; q++) {
-                    for (int32_t m = 0; ok && m < steps[q].n; m++) {
-                        ok = apart(t, nd, ls[static_cast<size_t>(steps[q].li[m])], layers[j]);
+            s.li[s.n++] = static_cast<int32_t>(at);
+            rd.clear();
+            wr.clear();
+            accesses(l);
+            int ch = 0;
+            SoftMaxCall sc;
+            EltOp eo[kConcatMax + 1];
+            bool link = false;
+            if (layer_at(at, &ch)) {
+                s.kind = kStepLayers;
+                s.li[s.n++] = static_cast<int32_t>(i);
+                f.key = ch;
+                // conv1's output is neither stored nor read
+                const int32_t h = cls[static_cast<size_t>(nd[l.first_node + l.n_nodes - 1].dst)];
+                wr.clear();
+                accesses(ls[i++]);
+                rd.erase(std::remove(rd.begin(), rd.end(), h), rd.end());
+            } else if (l.kind == CBX_GL_CONCAT) {
+                while (s.n < kConcatMax && appends(i)) s.li[s.n++] = static_cast<int32_t>(i++);
+                // the longest run of them that is plain copies
+                while (s.n > 1 && !(f.elts = concat_of(t, nd, ls, s.li, s.n, eo))) {
+                    s.n--;
+                    i--;
+                }
+                if (s.n == 1) f.elts = concat_of(t, nd, ls, s.li, 1, eo);
+                if (s.n > 1) {
+                    wr.clear();
+                    touch(&wr, nd[ls[i - 1].first_node].dst);
+                    for (int32_t m = 1; m < s.n; m++) touch(&rd, nd[ls[static_cast<size_t>(s.li[m])].first_node].src[1]);
+                }
+                if (f.elts) s.kind = kStepElt;
+            } else if (softmax_of(t, nd, l, st, &sc, &f.key)) {
+                s.kind = kStepSoftMax;
+            } else {
+                link = link_of(t, nd, l, &f.link);
+                // a scale or a mask product joins a chain it follows, but
+                // starts none: alone it is element-wise
+                if (link && l.kind != CBX_GL_SCALE && l.kind != CBX_GL_BINARY) s.kind = kStepRows;
+                else if ((f.elts = elt_of(t, nd, l, eo)) > 0) s.kind = kStepElt;
+            }
+            // one past the last step this one conflicts with
+            int32_t lo = -1;
+            for (int32_t c : rd) lo = std::max(lo, last_wr[static_cast<size_t>(c)]);
+            for (int32_t c : wr) lo = std::max(lo, std::max(last_wr[static_cast<size_t>(c)], last_rd[static_cast<size_t>(c)]));
+            const size_t from = static_cast<size_t>(lo + 1);
+            size_t to = steps.size();
+            if (link && from > 0 && steps[from - 1].kind == kStepRows && steps[from - 1].n < kStepMax &&
+                follows(from - 1, f.link)) {
+                to = from - 1;
+                info[to].link = f.link;
+                f.elts = 0;
+            } else if (s.kind == kStepLayers || s.kind == kStepElt || s.kind == kStepSoftMax) {
+                for (size_t q = from; q < steps.size(); q++) {
+                    const bool room = steps[q].n + s.n <= (s.kind == kStepLayers ? 2 * kResMax : kStepMax) &&
+                                      info[q].elts + f.elts <= kEltMax;
+                    if (steps[q].kind == s.kind && info[q].key == f.key && room) {
+                        to = q;
+                        break;
                     }
                 }
-                if (!ok) {
-                    j++;
-                    continue;
-                }
-                for (int32_t m = 0; m < 2; m++) steps[i].li[steps[i].n++] = steps[j].li[m];
-                steps.erase(steps.begin() + static_cast<std::ptrdiff_t>(j));
-                layers.erase(layers.begin() + static_cast<std::ptrdiff_t>(j));
             }
+            if (to == steps.size()) {
+                steps.push_back(s);
+                info.push_back(f);
+            } else {
+                for (int32_t m = 0; m < s.n; m++) steps[to].li[steps[to].n++] = s.li[m];
+                info[to].elts += f.elts;
+            }
+            const int32_t me = static_cast<int32_t>(to);
+            for (int32_t c : rd) last_rd[static_cast<size_t>(c)] = std::max(last_rd[static_cast<size_t>(c)], me);
+            for (int32_t c : wr) last_wr[static_cast<size_t>(c)] = std::max(last_wr[static_cast<size_t>(c)], me);
         }
         return steps;
     }
@@ -1326,35 +1773,113 @@ struct Scheduler {
 
 std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd, int32_t n,
                            const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep) {
-    Scheduler s{t, nd, ls, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
-                std::vector<char>(static_cast<size_t>(n_t), 0), {}};
+    int rc = CBX_OK;
+    const DeviceState* st = current_state(&rc);
+    if (!st) {   // the launches report it
+        std::vector<Step> one;
+        for (size_t i = 0; i < ls.size(); i++) {
+            Step s;
+            s.li[s.n++] = static_cast<int32_t>(i);
+            one.push_back(s);
+        }
+        return one;
+    }
+    Scheduler s{t, nd, ls, st, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
+                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}};
     for (int32_t k = 0; k < n_keep; k++) s.keep[static_cast<size_t>(keep[k])] = 1;
     for (int32_t i = 0; i < n; i++) {
         for (int32_t q : nd[i].src) {
             if (q >= 0) s.uses[static_cast<size_t>(q)]++;
         }
     }
-    return s.run();
+    return std::move(s.run(n_t));
+}
+
+// A chain's links as the kernel takes them, each operand from memory or
+// from the link before.
+RowLink row_link(const LinkT& k, const LinkT* prev) {
+    auto p = [](const cbx_tensor* t) { return t ? static_cast<const float*>(t->data) : nullptr; };
+    RowLink l{};
+    const uint32_t fa = prev && !k.a_vec ? Scheduler::from_chain(*prev, k.a) : kFromMemory;
+    const uint32_t fr = !k.r ? kAbsent : prev ? Scheduler::from_chain(*prev, k.r) : kFromMemory;
+    l.flags = fa << kLinkA | fr << kLinkR | (k.a_vec ? kLinkAVec : 0) | (k.ab ? kLinkBias : 0) |
+              (k.norm ? kLinkNorm : 0) | (k.mish ? kLinkMish : 0) | (k.mask ? kLinkMask : 0) | (k.scaled ? kLinkScale : 0);
+    l.a = fa == kFromMemory ? p(k.a) : nullptr;
+    l.r = fr == kFromMemory ? p(k.r) : nullptr;
+    l.ab = p(k.ab);
+    l.w = p(k.w);
+    l.b = p(k.b);
+    l.mask = p(k.mask);
+    l.s = k.store_s ? static_cast<float*>(k.s->data) : nullptr;
+    l.y = k.y ? static_cast<float*>(k.y->data) : nullptr;
+    l.eps = k.eps;
+    l.scale = k.scale;
+    return l;
 }
 
 // Issues a step.  *at names the planned launch an error belongs to.
 int run_step(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const std::vector<cbx_glaunch>& ls,
-             const Step& st, cbx_stream s, int32_t* at) {
+             const Step& st, cbx_stream stream, int32_t* at) {
     *at = st.li[0];
-    if (st.n == 1) return run(t, nd, n_nodes, ls[static_cast<size_t>(st.li[0])], s);
+    if (st.n == 1) return run(t, nd, n_nodes, ls[static_cast<size_t>(st.li[0])], stream);   // alone: its own kernel
     int rc = CBX_OK;
     DeviceState* ds = current_state(&rc);
     if (!ds) return rc;
-    ResLayer r[kResMax];
-    int ch = 0;
-    for (int32_t m = 0; m < st.n; m += 2) {
-        ConvCall c1, c2;
-        if (conv_call_of(t, nd, ls[static_cast<size_t>(st.li[m])], &c1) ||
-            conv_call_of(t, nd, ls[static_cast<size_t>(st.li[m + 1])], &c2) || !res_layer_of(c1, c2, &r[m / 2], &ch)) {
-            return set_error(CBX_ERR_INVALID_ARG, "a ResBlock layer changed under its schedule");
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    auto L = [&](int32_t m) -> const cbx_glaunch& { return ls[static_cast<size_t>(st.li[m])]; };
+    auto changed = [&]() { return set_error(CBX_ERR_INVALID_ARG, "a launch changed under its schedule"); };
+    switch (st.kind) {
+        case kStepLayers: {
+            ResLayer r[kResMax];
+            int ch = 0;
+            for (int32_t m = 0; m < st.n; m += 2) {
+                ConvCall c1, c2;
+                if (conv_call_of(t, nd, L(m), &c1) || conv_call_of(t, nd, L(m + 1), &c2) ||
+                    !res_layer_of(c1, c2, &r[m / 2], &ch)) {
+                    return changed();
+                }
+            }
+            return launch_res_layers(r, st.n / 2, ch, ds, s);
+        }
+        case kStepElt: {
+            EltOp e[kEltMax + kConcatMax + 1];
+            int n = 0;
+            for (int32_t m = 0; m < st.n;) {
+                int32_t c = 1;   // launches of one entry
+                int k;
+                if (L(m).kind == CBX_GL_CONCAT) {
+                    while (m + c < st.n && st.li[m + c] == st.li[m] + c && L(m + c).kind == CBX_GL_CONCAT &&
+                           nd[L(m + c).first_node].src[0] == nd[L(m + c - 1).first_node].dst) {
+                        c++;
+                    }
+                    k = concat_of(t, nd, ls, st.li + m, c, e + n);
+                } else {
+                    k = elt_of(t, nd, L(m), e + n);
+                }
+                if (k == 0 || n + k > kEltMax) return changed();
+                n += k;
+                m += c;
+            }
+            return launch_elt_group(e, n, ds, s);
+        }
+        case kStepSoftMax: {
+            SoftMaxCall c[kStepMax];
+            int64_t key;
+            for (int32_t m = 0; m < st.n; m++) {
+                if (!softmax_of(t, nd, L(m), ds, &c[m], &key)) return changed();
+            }
+            return launch_soft_max_group(c, st.n, ds, s);
+        }
+        default: {
+            RowLink r[kStepMax];
+            LinkT k[2];
+            for (int32_t m = 0; m < st.n; m++) {
+                if (!link_of(t, nd, L(m), &k[m & 1])) return changed();
+                r[m] = row_link(k[m & 1], m ? &k[(m & 1) ^ 1] : nullptr);
+            }
+            return launch_row_chain(r, st.n, k[0].ne0, k[0].nr, ds, s);
         }
     }
-    return launch_res_layers(r, st.n / 2, ch, ds, reinterpret_cast<hipStream_t>(s));
 }
 
 // The planned launches of a step that run something (views do not)

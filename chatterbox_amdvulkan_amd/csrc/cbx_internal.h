@@ -195,6 +195,54 @@ int conv1d_call(const ConvCall& c, cbx_stream stream);
 // Whether c1 then c2 are a ResBlock layer (c2 reads c1's output, which the
 // caller says nothing else reads) that one launch takes: *l is filled.
 bool res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int* ch);
+// ---- several launches of a node list in one kernel (k_group.hip) ------------
+// y = act((x op b) + b2) over n4 float4s, contiguous, 16-byte aligned.
+// How b runs against x: along its rows, a value a row (rows of whole float4s,
+// or of any length), as x itself.
+enum { kEltNone = 0, kEltVec = 1, kEltRow = 2, kEltFull = 3, kEltRowAny = 4 };
+constexpr int kEltScale = 1000;    // act: times param
+struct EltOp {
+    const float *x, *b, *b2;       // b2: a vector along ne0 of C2 floats, or null
+    float* y;
+    uint32_t n4;
+    uint32_t C, C2;                // kEltVec: floats of b; kEltRow: values of b
+    uint32_t ne0_4;                // float4s of an x row (kEltRow, ld4); its floats (kEltRowAny)
+    uint32_t ld4;                  // float4s from y row to y row when not contiguous, else 0
+    int32_t act;
+    float param;
+    int16_t bmode, mul;            // mul: x * b, else x + b
+};
+constexpr int kEltMax = 48;
+int launch_elt_group(const EltOp* ops, int n, DeviceState* st, hipStream_t s);
+// A link of a row chain: S = (a + ab) + r, stored to s; Y = LN(S) * w + b [->
+// mish] when norm, else S; then Y times the row's mask value and / or scale,
+// stored to y.  Rows contiguous, ne0 % 4 == 0, 16-byte aligned.
+enum { kAbsent = 0, kFromMemory = 1, kFromSum = 2, kFromResult = 3 };   // a and r: memory, or the last link's S or Y
+enum {
+    kLinkA = 0, kLinkR = 2,       // two bits each: where a and r come from
+    kLinkAVec = 1 << 4,           // a is one row, read by every row
+    kLinkBias = 1 << 5,           // ab is there
+    kLinkNorm = 1 << 6, kLinkMish = 1 << 7, kLinkMask = 1 << 8, kLinkScale = 1 << 9
+};
+struct RowLink {
+    const float *a, *ab, *r, *w, *b, *mask;
+    float *s, *y;
+    float eps, scale;
+    uint32_t flags, pad;
+};
+constexpr int kChainMax = 48;
+int launch_row_chain(const RowLink* ls, int n, int64_t ne0, int64_t nr, DeviceState* st, hipStream_t s);
+// Softmax calls that take one kernel of k_softmax.hip (equal non-negative
+// keys) side by side in a launch.
+struct SoftMaxCall {
+    const cbx_tensor *x, *b;
+    float scale;
+    int64_t n_past;
+    cbx_tensor* y;
+};
+constexpr int kSoftMaxGroup = 48;
+int64_t soft_max_group_key(const SoftMaxCall& c, const DeviceState* st);
+int launch_soft_max_group(const SoftMaxCall* c, int n, DeviceState* st, hipStream_t s);
 // Whether prepared weights were made from a weight of these extents: a
 // conv1d weight (K, C_in, C_out) when up == 0, else a transposed weight
 // (K, C_out, C_in) split for stride up.

@@ -98,7 +98,7 @@ __device__ __forceinline__ void store_v(char* p, float4 v) {
 // row and nothing waits (bounds check, block size) before the loads issue.
 // FLAT: rows at one stride each, so the row map's flag is not tested either.
 template <int NV, int WPB, bool FLAT, bool ADD, int VW>
-__global__ __launch_bounds__(64 * WPB) void k_soft_max_wave(SoftMaxArgs a) {
+__device__ __forceinline__ void sm_wave_rows(const SoftMaxArgs& a) {
     // every field in the first batch of argument loads (left alone, the
     // compiler loads the row count first and the rest after its test: a
     // second scalar round trip before the row loads)
@@ -162,6 +162,11 @@ __global__ __launch_bounds__(64 * WPB) void k_soft_max_wave(SoftMaxArgs a) {
             store_v<VW>(yr + c * 4, make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv));
         }
     }
+}
+
+template <int NV, int WPB, bool FLAT, bool ADD, int VW>
+__global__ __launch_bounds__(64 * WPB) void k_soft_max_wave(SoftMaxArgs a) {
+    sm_wave_rows<NV, WPB, FLAT, ADD, VW>(a);
 }
 
 // Few rows of up to 4096 scores at any alignment (the decode step's H
@@ -254,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void k_soft_max_row(SoftMaxArgs a) {
 // butterflies -- no LDS and no barrier.  One kernel for every length up to
 // 1024, like k_soft_max_row.
 template <bool FLAT, bool ADD>
-__global__ __launch_bounds__(WAVE) void k_soft_max_row_w(SoftMaxArgs a) {
+__device__ __forceinline__ void sm_row_w(const SoftMaxArgs& a) {
     constexpr int K = 1024 / WAVE;
     arg_now(a.x); arg_now(a.y); arg_now(reinterpret_cast<const void*>(a.mx.nb1));
     arg_now(reinterpret_cast<const void*>(a.my.nb1)); arg_now(reinterpret_cast<const void*>(a.n_past));
@@ -307,6 +312,53 @@ __global__ __launch_bounds__(WAVE) void k_soft_max_row_w(SoftMaxArgs a) {
         const int c = lane + k * WAVE;
         if (k < nk && c < ne0) yr[c] = v[k] * inv;
     }
+}
+
+template <bool FLAT, bool ADD>
+__global__ __launch_bounds__(WAVE) void k_soft_max_row_w(SoftMaxArgs a) {
+    sm_row_w<FLAT, ADD>(a);
+}
+
+// Calls of one kernel side by side (grid y): a node list's softmaxes that do
+// not depend on each other.  Rows at one stride each, the same row count.
+struct SmFlat {
+    const char *x, *b, *y;
+    int64_t nb1x, nb1b, nb1y, n_past;
+    int32_t ne0;
+    uint32_t n_q;
+    float s;
+};
+struct SmGroup {
+    int32_t nr;
+    SmFlat c[kSoftMaxGroup];
+};
+static_assert(sizeof(SmGroup) <= 4096, "softmax group arguments must fit the kernel argument segment");
+
+__device__ __forceinline__ SoftMaxArgs sm_of(const SmGroup& g) {
+    const SmFlat& c = g.c[blockIdx.y];
+    SoftMaxArgs a{};
+    a.x = c.x;
+    a.b = c.b;
+    a.y = const_cast<char*>(c.y);
+    a.mx.nb1 = c.nb1x;
+    a.mb.nb1 = c.nb1b;
+    a.my.nb1 = c.nb1y;
+    a.n_past = c.n_past;
+    a.ne0 = c.ne0;
+    a.nr = g.nr;
+    a.n_q = c.n_q;
+    a.s = c.s;
+    return a;
+}
+
+template <int NV, int WPB, bool ADD, int VW>
+__global__ __launch_bounds__(64 * WPB) void k_soft_max_wave_n(SmGroup g) {
+    sm_wave_rows<NV, WPB, true, ADD, VW>(sm_of(g));
+}
+
+template <bool ADD>
+__global__ __launch_bounds__(WAVE) void k_soft_max_row_w_n(SmGroup g) {
+    sm_row_w<true, ADD>(sm_of(g));
 }
 
 // Any row length: max, then the f64 sum of exponentials, then the output,
@@ -368,11 +420,16 @@ void sm_wave(int nv, const SoftMaxArgs& a, hipStream_t strm) {
     }
 }
 
+// the wave-per-row kernel's vectors a lane
+int sm_nv(int64_t ne0, int vw) {
+    const int64_t need = cdiv(ne0, 64 * vw);
+    return need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : 16;
+}
+
 // the wave-per-row kernel for rows of VW-float vectors (NV of them a lane)
 template <bool ADD, int VW>
 void sm_waves(const SoftMaxArgs& a, int64_t ne0, const DeviceState* st, hipStream_t strm) {
-    const int64_t need = cdiv(ne0, 64 * VW);
-    const int nv = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : 16;
+    const int nv = sm_nv(ne0, VW);
     // strided-plane layouts take one row per workgroup through the row map
     if (!(a.mx.flat && a.my.flat && (!ADD || a.mb.flat))) sm_wave<1, false, ADD, VW>(nv, a, strm);
     else if (waves_for(a.nr, st) == 1) sm_wave<1, true, ADD, VW>(nv, a, strm);
@@ -420,6 +477,48 @@ bool vec_rows(const cbx_tensor* t, size_t al) {
            (t->ne[3] <= 1 || t->nb[3] % al == 0);
 }
 
+template <int WPB, bool ADD, int VW>
+void sm_wave_group(int nv, const SmGroup& g, dim3 grid, hipStream_t strm) {
+    const dim3 block(64 * WPB);
+    switch (nv) {
+        case 1: hipLaunchKernelGGL((k_soft_max_wave_n<1, WPB, ADD, VW>), grid, block, 0, strm, g); break;
+        case 2: hipLaunchKernelGGL((k_soft_max_wave_n<2, WPB, ADD, VW>), grid, block, 0, strm, g); break;
+        case 4: hipLaunchKernelGGL((k_soft_max_wave_n<4, WPB, ADD, VW>), grid, block, 0, strm, g); break;
+        case 8: hipLaunchKernelGGL((k_soft_max_wave_n<8, WPB, ADD, VW>), grid, block, 0, strm, g); break;
+        default: hipLaunchKernelGGL((k_soft_max_wave_n<16, WPB, ADD, VW>), grid, block, 0, strm, g); break;
+    }
+}
+
+template <bool ADD>
+void sm_group(int vw, int nv, int wpb, const SmGroup& g, int n, hipStream_t strm) {
+    const dim3 grid(static_cast<unsigned>(cdiv(g.nr, wpb)), static_cast<unsigned>(n));
+    if (vw == 0) hipLaunchKernelGGL((k_soft_max_row_w_n<ADD>), grid, dim3(WAVE), 0, strm, g);
+    else if (vw == 4 && wpb == 1) sm_wave_group<1, ADD, 4>(nv, g, grid, strm);
+    else if (vw == 4) sm_wave_group<4, ADD, 4>(nv, g, grid, strm);
+    else if (wpb == 1) sm_wave_group<1, ADD, 2>(nv, g, grid, strm);
+    else sm_wave_group<4, ADD, 2>(nv, g, grid, strm);
+}
+
+// The kernel sm_launch takes for a call of uniformly strided rows: vw 0 for
+// the one-wave row kernel, else the vector width of the wave-per-row one;
+// false for the others.
+bool sm_kernel(const SoftMaxCall& c, const DeviceState* st, int* vw, int* nv, int* wpb) {
+    const int64_t nr = nrows(c.x), ne0 = c.x->ne[0];
+    if (nr >= (int64_t{1} << 31) || !flat_rows(c.x) || !flat_rows(c.y) || (c.b && !flat_rows(c.b))) return false;
+    const bool few = ne0 <= kWaveMaxRow && nr < int64_t{4} * st->n_cu;
+    auto rows = [&](size_t al) { return vec_rows(c.x, al) && vec_rows(c.y, al) && (!c.b || vec_rows(c.b, al)); };
+    *vw = 0;
+    *nv = *wpb = 1;
+    if (!few && ne0 <= kWaveMaxRow && ne0 % 4 == 0 && rows(16)) *vw = 4;
+    else if (!few && ne0 <= kWaveMaxRow / 2 && ne0 % 2 == 0 && rows(8)) *vw = 2;
+    else if (ne0 > 1024) return false;
+    if (*vw) {
+        *nv = sm_nv(ne0, *vw);
+        *wpb = waves_for(nr, st);
+    }
+    return true;
+}
+
 }  // namespace
 
 int launch_soft_max(const cbx_tensor* x, const cbx_tensor* b, float s, int64_t n_past, cbx_tensor* y,
@@ -438,6 +537,32 @@ int launch_soft_max(const cbx_tensor* x, const cbx_tensor* b, float s, int64_t n
         sm_launch<false>(a, ne0, vec, vec2, view_of(x), vb, view_of(y), flat_rows(x), false, flat_rows(y), st, strm);
     }
     return check_launch("soft_max");
+}
+
+// Calls with one key run in one kernel: the row count and the kernel.
+int64_t soft_max_group_key(const SoftMaxCall& c, const DeviceState* st) {
+    int vw, nv, wpb;
+    if (!sm_kernel(c, st, &vw, &nv, &wpb)) return -1;
+    return (nrows(c.x) << 16) | (vw << 12) | (wpb << 8) | (nv << 1) | (c.b ? 1 : 0);
+}
+
+int launch_soft_max_group(const SoftMaxCall* c, int n, DeviceState* st, hipStream_t strm) {
+    int vw, nv, wpb;
+    if (n < 1 || n > kSoftMaxGroup || !sm_kernel(c[0], st, &vw, &nv, &wpb)) {
+        return set_error(CBX_ERR_INVALID_ARG, "soft_max: not a group of one kernel");
+    }
+    SmGroup g;
+    g.nr = static_cast<int32_t>(nrows(c[0].x));
+    for (int i = 0; i < n; i++) {
+        const cbx_tensor *x = c[i].x, *b = c[i].b ? c[i].b : c[i].x, *y = c[i].y;
+        g.c[i] = SmFlat{static_cast<const char*>(x->data), static_cast<const char*>(b->data),
+                        static_cast<const char*>(y->data), static_cast<int64_t>(x->nb[1]), static_cast<int64_t>(b->nb[1]),
+                        static_cast<int64_t>(y->nb[1]), c[i].n_past, static_cast<int32_t>(x->ne[0]),
+                        static_cast<uint32_t>(x->ne[1] > 0 ? x->ne[1] : 1), c[i].scale};
+    }
+    if (c[0].b) sm_group<true>(vw, nv, wpb, g, n, strm);
+    else sm_group<false>(vw, nv, wpb, g, n, strm);
+    return check_launch("soft_max_group");
 }
 
 }  // namespace cbx

@@ -267,12 +267,32 @@ def _ready(t: torch.Tensor):
 _DTYPES = {torch.float32: F32, torch.float16: F16, torch.int32: I32}
 
 
+# What desc() fills in besides the address depends on the shape, strides and
+# types alone: the filled descriptor of each layout met (9 descriptors of a
+# causal block's two calls: 36 us of host time without, 16 with it).
+_layouts: dict = {}
+_LAYOUTS_MAX = 4096
+
+
 def desc(t: torch.Tensor, ggml_type: Optional[int] = None) -> Tensor:
     """cbx_tensor for a torch tensor (up to 4 dims, any strides)."""
+    key = (t.shape, t.stride(), t.dtype, ggml_type)
+    raw = _layouts.get(key)
+    if raw is None:
+        raw = bytes(_layout(t, ggml_type))
+        if len(_layouts) >= _LAYOUTS_MAX:
+            _layouts.clear()
+        _layouts[key] = raw
+    d = Tensor.from_buffer_copy(raw)
+    d.data = t.data_ptr()
+    return d
+
+
+def _layout(t: torch.Tensor, ggml_type: Optional[int]) -> Tensor:
+    """The descriptor of t with a null address."""
     if t.dim() > 4:
         raise CbxError(ERR_INVALID_ARG, "more than 4 dims")
     d = Tensor()
-    d.data = t.data_ptr()
     es = t.element_size()
     shape = list(t.shape[::-1]) or [1]
     if t.numel() == 0:
@@ -308,7 +328,15 @@ def _ref(d: Optional[Tensor]):
     return ctypes.byref(d) if d is not None else None
 
 
+# The current stream's handle straight from torch's C++ side where this
+# torch has it (0.3 us against 2.5 for the Stream object).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> ctypes.c_void_p:
+    if _raw_stream is not None and _raw_device is not None and torch.cuda.is_initialized():
+        return ctypes.c_void_p(_raw_stream(_raw_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 

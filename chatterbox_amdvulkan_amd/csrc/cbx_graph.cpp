@@ -2223,12 +2223,20 @@ static int update_changed(cbx_graph_exec* x, GraphInst& t, const cbx_tensor* ten
             changed.push_back(static_cast<int32_t>(i));
         }
     }
-    if (!changed.empty()) {
+    if (changed.empty()) {
+        const int rc = wait_marks(x, f);
+        if (rc) return rc;
+        if (const int r2 = mark_launches(x, f)) return r2;
+    } else {
         hipGraph_t g = nullptr;
         std::vector<int32_t> kcount;
         int32_t issued = 0;
         int rc = record(tensors, nodes, n_nodes, ls, steps, &changed, x->cs, &g, &kcount, &issued, f);
         if (rc) return rc;   // t untouched
+        if ((rc = wait_marks(x, f)) || (rc = mark_launches(x, f))) {
+            (void)hipGraphDestroy(g);
+            return rc;
+        }
         std::vector<hipGraphNode_t> gn;
         bool ok = kernel_chain(g, &gn);
         size_t want = 0;
@@ -2295,10 +2303,16 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
         std::vector<uint64_t> sig;
         std::vector<size_t> sig_at;
         signatures(tensors, nodes, ls, steps, &sig, &sig_at);
+        // the list the current instantiation already holds: nothing to set
+        const GraphInst& c = exec->inst[exec->cur];
+        if (c.indexed && c.steps == steps && c.sig == sig && c.ls.size() == ls.size()) {
+            if (n_launches) *n_launches = c.n_launches;
+            if (in_place) *in_place = 1;
+            return CBX_OK;
+        }
         // the instantiation to re-point is the one not replayed since the
-        // last update: wait for its replays (issued before that update),
-        // then mark the current one's
-        if ((rc = wait_marks(exec, f)) || (rc = mark_launches(exec, f))) return rc;
+        // last update: update_changed records first, waits for its replays
+        // (issued before that update) and marks the current one's, then sets
         bool done = false;
         if ((rc = update_changed(exec, t, tensors, nodes, n_nodes, ls, steps, sig, sig_at, &done, f))) return rc;
         if (done) {

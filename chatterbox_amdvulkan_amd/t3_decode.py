@@ -28,6 +28,8 @@ live in device int32 tensors the caller writes.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -35,6 +37,11 @@ from . import cbxops as C
 
 BLOCK_IN = ("ln1_w", "ln1_b", "qkv_b", "out_b", "ln2_w", "ln2_b", "fc_b", "proj_b",
             "qkv_mm", "kq", "out_mm", "fc_mm", "proj_mm")
+# the fields of a descriptor and a node that a token changes
+TENSOR_FIELDS = np.dtype({"names": ["ne", "nb"], "formats": [(np.int64, 4), (np.uint64, 4)],
+                          "offsets": [C.Tensor.ne.offset, C.Tensor.nb.offset], "itemsize": ctypes.sizeof(C.Tensor)})
+NODE_FIELDS = np.dtype({"names": ["iparam"], "formats": [np.int32], "offsets": [C.GNode.iparam.offset],
+                        "itemsize": ctypes.sizeof(C.GNode)})
 BLOCK_OUT = ("ln1", "qkv", "probs", "attn_res", "ln2", "gelu", "h")
 
 
@@ -133,6 +140,8 @@ class T3DecodeStep:
         keep += [h0, y]
         g.bind_arrays(keep)
         self.graph, self.keep, self.n_past = g, keep, n_past
+        self._score_ids = np.array([i for ids in self._kq_ids for i in ids])
+        self._views = None
 
     def retarget(self, n_past: int) -> None:
         """The list of the token after n_past cached ones: the score views
@@ -142,18 +151,20 @@ class T3DecodeStep:
         if not 0 <= n_past < self.max_ctx:
             raise ValueError(f"n_past {n_past} outside [0, {self.max_ctx})")
         n_kv = n_past + 1
-        g = self.graph
-        row, plane = 4 * n_kv, 4 * n_kv * self.n_head
-        for ids in self._kq_ids:
-            for i in ids:
-                d = g._descs[i]
-                d.ne[0] = n_kv
-                d.nb[1] = row
-                d.nb[2] = row
-                d.nb[3] = plane
-        for k in self._mask_nodes:
-            g.nodes[k].iparam = n_past
+        t, n = self._arrays()
+        ids = self._score_ids
+        t["ne"][ids, 0] = n_kv
+        t["nb"][ids, 1:3] = 4 * n_kv
+        t["nb"][ids, 3] = 4 * n_kv * self.n_head
+        n["iparam"][self._mask_nodes] = n_past
         self.n_past = n_past
+
+    def _arrays(self):
+        """The bound descriptor and node arrays as numpy records."""
+        T, N, _ = self.graph._arrays(self.keep)
+        if self._views is None or self._views[0] is not T:
+            self._views = (T, np.frombuffer(T, TENSOR_FIELDS), np.frombuffer(N, NODE_FIELDS))
+        return self._views[1:]
 
     def set_token(self, token: int, position: int) -> None:
         """Writes the token id and its position into their device tensors

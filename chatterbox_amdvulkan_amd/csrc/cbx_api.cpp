@@ -1303,7 +1303,7 @@ int cbx_conv_transpose1d(const cbx_tensor* x, const cbx_conv1d_weights* w, int p
     return launch_conv1d(x, w->data, w->taps, w->c_in_pad, w->c_out, 1, up == 1 ? static_cast<int>(w->k) - 1 - pad : 0,
                          1, up, pad, w->w_ph, prologue, prologue == CBX_CONV_PRO_SNAKE ? alpha : nullptr,
                          prologue == CBX_CONV_PRO_SNAKE ? alpha_inv : nullptr, slope, bias, nullptr, y, st,
-                         reinterpret_cast<hipStream_t>(stream));
+                         reinterpret_cast<hipStream_t>(stream), nullptr, 1.0f, static_cast<int>(w->k));
 }
 
 int cbx_causal_conv1d(const cbx_tensor* x, const cbx_conv1d_weights* w, const cbx_tensor* mask,

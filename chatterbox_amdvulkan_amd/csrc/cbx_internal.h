@@ -152,14 +152,15 @@ constexpr int kConvProMask = 3;
 // (K, C_in, C_out); up >= 1: transposed weight (K, C_out, C_in) split into
 // max(up, 1) phases of `taps` taps), and the conv itself (up > 1: the
 // transposed conv's phases, crop outputs cut from each end, w_ph halves of
-// weights per phase).
+// weights per phase, w_taps the weight's taps over all phases).
 int conv1d_weights_layout(int64_t c_in, int64_t c_out, int64_t* c_in_pad, int64_t* c_out_pad);
 int launch_conv1d_weights(const cbx_tensor* w, int up, int64_t taps, _Float16* out, int64_t c_in_pad,
                           int64_t c_out_pad, hipStream_t s);
 int launch_conv1d(const cbx_tensor* x, const _Float16* w16, int64_t k, int64_t c_in_pad, int64_t c_out, int stride,
                   int pad, int dil, int up, int crop, int64_t w_ph, int pro, const cbx_tensor* alpha,
                   const cbx_tensor* alpha_inv, float slope, const cbx_tensor* bias, const cbx_tensor* res, cbx_tensor* y,
-                  DeviceState* st, hipStream_t s, const cbx_tensor* acc = nullptr, float oscale = 1.0f);
+                  DeviceState* st, hipStream_t s, const cbx_tensor* acc = nullptr, float oscale = 1.0f,
+                  int w_taps = 0);
 // One ResBlock layer run by k_resblock.hip: y = res + conv2(snake2(conv1(
 // snake1(x)) + b1)) + b2, then [+ acc [* oscale]], all (ch, T) f32 with
 // 16-byte aligned rows at the given byte steps; both convs stride 1 with

@@ -27,8 +27,9 @@
 // it instead of all reading the same KiB.  The finished tile goes through
 // LDS to row-contiguous float4 stores (with the bias and residual reads).
 //
-// The transposed conv of the upsamplers (hift_vocoder.cpp:96-115) runs on
-// the same kernel: output phase ph of stride s is a stride-1 conv of the
+// The transposed conv of the upsamplers (hift_vocoder.cpp:96-115) has a
+// kernel of its own (k_conv_up) for whole channel blocks; any other runs on
+// the same kernel as the conv: output phase ph of stride s is a stride-1 conv of the
 // input with that phase's taps reversed, so the s phases are s such convs
 // side by side in grid z, each writing every s-th output row.
 //
@@ -798,6 +799,131 @@ __global__ __launch_bounds__(kPipeThreads) __attribute__((amdgpu_waves_per_eu(OC
     }
 }
 
+// ---- transposed conv ----------------------------------------------------------
+// The upsamplers (stride up > 1) write up times their input: what bounds them
+// is that traffic.  k_conv1d runs the up phases as convs of their own, each
+// staging the input again and writing every up-th row.  Here a workgroup
+// stages the activated f16 window of MT*32 output steps u (up output frames
+// each) once, and its W waves each compute one (phase, 32 channels) tile of
+// them over all taps and input channels: the phases of a step are read from
+// one window and their rows written together.  A wave's weights are one
+// contiguous run of fragments, read eight steps ahead; the operands are swapped
+// (weights A, window rows B), so that a lane stores four channels of a frame.
+// Frames a phase's zero-padded first tap would reach are skipped with it.
+template <int PRO, int MT, int W>
+__global__ __launch_bounds__(64 * W) void k_conv_up(ConvArgs a, int pad_max) {
+    extern __shared__ _Float16 lds[];   // [a.win][c_in + 8]
+    constexpr int M = MT * 32, NTH = 64 * W, PF = 8;   // c_in % 128 == 0: whole groups of PF steps a tap
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned L = blockIdx.x, n_wg = gridDim.x;
+    const unsigned q8 = n_wg >> 3, r8 = n_wg & 7, xcd = L & 7, j8 = L >> 3;
+    const unsigned w = xcd < r8 ? xcd * (q8 + 1) + j8 : r8 * (q8 + 1) + (xcd - r8) * q8 + j8;
+    // tile groups of one window first: they meet in an XCD's L2
+    const int tg = static_cast<int>(w % static_cast<unsigned>(a.n_ct));
+    const unsigned wr = w / static_cast<unsigned>(a.n_ct);
+    const int ut = static_cast<int>(wr % static_cast<unsigned>(a.n_tt)), bz = static_cast<int>(wr / static_cast<unsigned>(a.n_tt));
+    const int u0 = ut * M, base_t = u0 - pad_max, cs = a.c_in + 8;
+    const int nco = a.c_out >> 5, tile = tg * W + wave;
+    const bool live = tile < a.up * nco;             // the last group may have idle waves
+    const int ph = live ? tile / nco : 0, ct = live ? tile - ph * nco : 0;
+    const int c1 = ((ph - a.crop) % a.up + a.up) % a.up;          // the phase's first output frame
+    const int pad = a.k - 1 - (c1 + a.crop - ph) / a.up;
+    // a.kch: the weight's taps.  A phase without any (K < up) sums nothing.
+    const bool pad_tap = ph + (a.k - 1) * a.up >= a.kch;
+    const int kp0 = pad_tap && a.k > 1 ? 1 : 0;
+    const int nb = a.c_in / kBlk, n_steps = pad_tap && a.k == 1 ? 0 : (a.k - kp0) * nb;
+    const int lo = lane * 8;
+    const _Float16* wp = a.w + ph * a.w_ph + (static_cast<int64_t>(ct) * a.k + kp0) * nb * 512 + lo;
+    half8 ring[PF];
+#pragma unroll
+    for (int j = 0; j < PF; j++) ring[j] = *reinterpret_cast<const half8*>(wp + j * 512);
+
+    {
+        const char* xb = a.x + static_cast<int64_t>(bz) * a.x_nb2;
+        const unsigned gpr = static_cast<unsigned>(a.c_in) >> 2, total = static_cast<unsigned>(a.win) * gpr;
+        constexpr int KST = 8;
+        for (unsigned e0 = tid; e0 < total; e0 += KST * NTH) {
+            float4 v[KST];
+            int off[KST];
+#pragma unroll
+            for (int i = 0; i < KST; i++) {
+                const unsigned e = e0 + i * NTH, r = e / gpr, cg = 4 * (e - r * gpr);
+                const int ti = base_t + static_cast<int>(r);
+                const bool in = e < total, ok = in && ti >= 0 && ti < a.t_in;
+                off[i] = in ? static_cast<int>(r) * cs + static_cast<int>(cg) : -1;
+                // rows outside x read row 0 and are zeroed (leaky(0) = 0)
+                const float4 t = *reinterpret_cast<const float4*>(xb + static_cast<int64_t>(ok ? ti : 0) * a.x_nb1 +
+                                                                  static_cast<int64_t>(in ? cg : 0) * 4);
+                v[i] = ok ? t : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int i = 0; i < KST; i++) {
+                if (off[i] < 0) continue;
+                half4 hv;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    hv[q] = static_cast<_Float16>(PRO == PRO_LEAKY ? act_leaky(get(v[i], q), a.slope) : get(v[i], q));
+                }
+                *reinterpret_cast<half4*>(lds + off[i]) = hv;
+            }
+        }
+    }
+    __syncthreads();
+    if (!live) return;
+
+    const int lrow = lane & 31, co0 = ct * 32 + 4 * (lane >> 5);   // accumulator 4g + q: channel co0 + 8g + q
+    floatx16 acc[MT];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const float4 b4 = a.bias ? *reinterpret_cast<const float4*>(a.bias + co0 + 8 * g) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[mt][4 * g + q] = get(b4, q);
+        }
+    }
+    int arow[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) arow[mt] = (mt * 32 + lrow + pad_max - pad + kp0) * cs + 8 * (lane >> 5);
+    half8 bv[2][MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) bv[0][mt] = *reinterpret_cast<const half8*>(lds + arow[mt]);
+    int aoff = 0, b = 0;   // of the group's first step
+    for (int s = 0; s < n_steps; s += PF) {
+        const bool last = s + PF >= n_steps;
+        const bool wrap = b + PF == nb;
+        const int an = last ? aoff : aoff + 16 * PF + (wrap ? 8 : 0);   // a tap's end: the next row, (c_in + 8) - 16 nb further
+        const _Float16* wn = last ? wp : wp + PF * 512;
+#pragma unroll
+        for (int j = 0; j < PF; j++) {
+            const int o = j + 1 < PF ? aoff + (j + 1) * 16 : an;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) bv[(j & 1) ^ 1][mt] = *reinterpret_cast<const half8*>(lds + arow[mt] + o);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ring[j], bv[j & 1][mt], acc[mt], 0, 0, 0);
+            }
+            ring[j] = *reinterpret_cast<const half8*>(wn + j * 512);
+        }
+        wp = wn;
+        aoff = an;
+        b = wrap ? 0 : b + PF;
+    }
+    char* yb = a.y + static_cast<int64_t>(bz) * a.y_nb2;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const int64_t t = c1 + static_cast<int64_t>(a.up) * (u0 + mt * 32 + lrow);
+        if (t < a.t_out) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                *reinterpret_cast<float4*>(yb + t * a.y_nb1 + static_cast<int64_t>(co0 + 8 * g) * 4) =
+                    make_float4(acc[mt][4 * g], acc[mt][4 * g + 1], acc[mt][4 * g + 2], acc[mt][4 * g + 3]);
+            }
+        }
+    }
+}
+
 // Fragment-major f16 copy of a conv weight, zero padded: fragment (phase,
 // co tile, tap, 16-channel block) is 64 lanes x 8 halves, lane l holding
 // w[co_tile*32 + l%32][block*16 + 8*(l/32) + j] at that tap -- one MFMA B
@@ -842,8 +968,8 @@ struct Tile {
     int bc() const { return wn * nt * 32; }
 };
 
-template <typename K>
-void conv_launch(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, const ConvArgs& a) {
+template <typename K, typename... More>
+void conv_launch(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, const ConvArgs& a, More... more) {
     // windows past 64 KiB use the larger LDS of gfx950 (160 KiB per
     // workgroup): raise the limit of each kernel once per device (every
     // instantiation has the same function type, so the record is keyed on
@@ -861,7 +987,7 @@ void conv_launch(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, con
             raised.insert({dev, fn});
         }
     }
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, a);
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, a, more...);
 }
 
 // (VEC, PF) in {(1, 4), (1, 2), (0, 2)}: unaligned rows take the shorter ring
@@ -937,7 +1063,7 @@ int launch_conv1d_weights(const cbx_tensor* w, int up, int64_t taps, _Float16* o
 int launch_conv1d(const cbx_tensor* x, const _Float16* w16, int64_t k, int64_t c_in_pad, int64_t c_out, int stride,
                   int pad, int dil, int up, int crop, int64_t w_ph, int pro, const cbx_tensor* alpha,
                   const cbx_tensor* alpha_inv, float slope, const cbx_tensor* bias, const cbx_tensor* res, cbx_tensor* y,
-                  DeviceState* st, hipStream_t s, const cbx_tensor* acc, float oscale) {
+                  DeviceState* st, hipStream_t s, const cbx_tensor* acc, float oscale, int w_taps) {
     ConvArgs a;
     a.x = static_cast<const char*>(x->data);
     a.w = w16;
@@ -1040,6 +1166,51 @@ int launch_conv1d(const cbx_tensor* x, const _Float16* w16, int64_t k, int64_t c
                 default: CBX_PIPE(PRO_NONE); break;
             }
 #undef CBX_PIPE
+            return check_launch("conv1d");
+        }
+    }
+    // transposed convs of 128 or 256 channels with aligned rows, without
+    // Snake, that give every CU two tiles of 32 steps: all phases from one
+    // staged window.  Fewer tiles, or a longer reduction a wave (512 -> 256
+    // channels), are latency: k_conv1d's split of the reduction is the faster
+    // (us, this against k_conv1d: 128 x 20000 12.3 / 20.0, 128 x 5000 5.9 /
+    // 7.2, 128 x 1000 5.5 / 4.9, 256 x 4000 14.1 / 17.3, 256 x 1000 7.3 /
+    // 8.9, 256 x 400 7.1 / 6.9, 512 x 500 12.1 / 11.9, 512 x 125 10.6 / 7.3)
+    const int64_t up_tiles = up > 1 ? cdiv(cdiv(a.t_out, up), 32) * up * (c_out / 32) * x->ne[2] : 0;
+    if (up > 1 && (pro == PRO_NONE || pro == PRO_LEAKY) && !res && !acc && a.c_in % 128 == 0 && a.c_in <= 256 &&
+        c_out % 32 == 0 && up_tiles >= int64_t{2} * st->n_cu) {
+        auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+        const bool one = x->ne[2] <= 1;
+        int pad_max = 0, pad_min = INT32_MAX;
+        for (int ph = 0; ph < up; ph++) {
+            const int c1 = ((ph - crop) % up + up) % up, pd = static_cast<int>(k) - 1 - (c1 + crop - ph) / up;
+            pad_max = std::max(pad_max, pd);
+            pad_min = std::min(pad_min, pd);
+        }
+        const int64_t tiles = up * (c_out / 32), steps = cdiv(a.t_out, up);
+        // a wave a tile; 64 steps a workgroup when that gives every CU one
+        const int wv = tiles % 6 == 0 ? 6 : 4;
+        const int64_t groups = cdiv(tiles, wv);
+        const int mt = cdiv(steps, 64) * groups * x->ne[2] >= st->n_cu ? 2 : 1;
+        const int64_t win = mt * 32 + k - 1 + pad_max - pad_min, items = cdiv(steps, mt * 32) * groups * x->ne[2];
+        const size_t lds = static_cast<size_t>(win) * static_cast<size_t>(a.c_in + 8) * sizeof(_Float16);
+        if (al16(a.x) && a.x_nb1 % 16 == 0 && (one || a.x_nb2 % 16 == 0) && al16(a.y) && a.y_nb1 % 16 == 0 &&
+            (one || a.y_nb2 % 16 == 0) && (!a.bias || al16(a.bias)) && lds <= kLdsMax && items < (int64_t{1} << 31)) {
+            a.win = static_cast<int32_t>(win);
+            a.kch = w_taps;
+            a.n_tt = static_cast<int32_t>(cdiv(steps, mt * 32));
+            a.n_ct = static_cast<int32_t>(groups);
+            const dim3 grid(static_cast<unsigned>(items)), block(64 * wv);
+#define CBX_UP(P)                                                                                   \
+    do {                                                                                            \
+        if (wv == 6 && mt == 2) conv_launch(k_conv_up<P, 2, 6>, grid, block, lds, s, a, pad_max);   \
+        else if (wv == 6) conv_launch(k_conv_up<P, 1, 6>, grid, block, lds, s, a, pad_max);         \
+        else if (mt == 2) conv_launch(k_conv_up<P, 2, 4>, grid, block, lds, s, a, pad_max);         \
+        else conv_launch(k_conv_up<P, 1, 4>, grid, block, lds, s, a, pad_max);                      \
+    } while (0)
+            if (pro == PRO_LEAKY) CBX_UP(PRO_LEAKY);
+            else CBX_UP(PRO_NONE);
+#undef CBX_UP
             return check_launch("conv1d");
         }
     }

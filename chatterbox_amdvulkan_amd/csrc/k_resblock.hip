@@ -308,6 +308,9 @@ template <int CH> struct ResTile;
 template <> struct ResTile<64> { static constexpr int MT = 2, WM = 2, WN = 2, PF = 4, M = 128; };
 template <> struct ResTile<128> { static constexpr int MT = 2, WM = 1, WN = 4, PF = 8, M = 64; };
 template <> struct ResTile<256> { static constexpr int MT = 1, WM = 1, WN = 8, PF = 8, M = 32; };
+// 256 channels, when 32-frame tiles are more than 1.5 a CU (the layers of
+// three ResBlocks side by side): 64-frame tiles read each weight half as often
+struct ResTileWide { static constexpr int MT = 2, WM = 1, WN = 8, PF = 16, M = 64; };
 
 static int64_t res_rows(int ch) {
     return ch == 64 ? ResTile<64>::M : ch == 128 ? ResTile<128>::M : ch == 256 ? ResTile<256>::M : 0;
@@ -340,9 +343,8 @@ bool res_layer_fits(const ResLayer& l, int ch, const DeviceState* st) {
     return (k > 14 ? 3 : 8) * tiles >= n_cu;
 }
 
-template <int CH>
+template <typename R, int CH>
 static void res_launch(uint32_t grid, size_t lds, hipStream_t s, const ResArgs& a) {
-    using R = ResTile<CH>;
     static_assert(R::M == R::WM * R::MT * 32, "tile rows");
     hipLaunchKernelGGL((k_res_layer<CH, R::MT, 1, R::WM, R::WN, R::PF>), dim3(grid), dim3(64 * R::WM * R::WN), lds, s, a);
 }
@@ -352,16 +354,24 @@ int launch_res_layers(const ResLayer* ls, int n, int ch, DeviceState* st, hipStr
     a.n = n;
     uint32_t at = 0;
     size_t lds = 0;
+    int64_t m = res_rows(ch), tiles = 0;
+    for (int i = 0; i < n; i++) tiles += res_tiles(ls[i], m);
+    if (ch == 256 && 2 * tiles > int64_t{3} * st->n_cu) {
+        bool fits = true;
+        for (int i = 0; i < n; i++) fits = fits && res_lds(ls[i], ch, ResTileWide::M) <= 64 * 1024;
+        if (fits) m = ResTileWide::M;
+    }
     for (int i = 0; i < n; i++) {
         a.l[i] = ls[i];
-        a.l[i].tiles = static_cast<int32_t>(res_tiles(ls[i], res_rows(ch)));
+        a.l[i].tiles = static_cast<int32_t>(res_tiles(ls[i], m));
         a.first[i] = at;
         at += static_cast<uint32_t>(cdiv(a.l[i].tiles, 8) * 8);
-        lds = std::max(lds, res_lds(ls[i], ch, res_rows(ch)));
+        lds = std::max(lds, res_lds(ls[i], ch, m));
     }
-    if (ch == 64) res_launch<64>(at, lds, s, a);
-    else if (ch == 128) res_launch<128>(at, lds, s, a);
-    else res_launch<256>(at, lds, s, a);
+    if (ch == 64) res_launch<ResTile<64>, 64>(at, lds, s, a);
+    else if (ch == 128) res_launch<ResTile<128>, 128>(at, lds, s, a);
+    else if (m == ResTileWide::M) res_launch<ResTileWide, 256>(at, lds, s, a);
+    else res_launch<ResTile<256>, 256>(at, lds, s, a);
     return check_launch("res_layers");
 }
 

@@ -783,7 +783,12 @@ int cbx_graph_launch(const cbx_tensor* tensors, int32_t n_tensors,
 
 /* Plans and runs the whole node list on `stream`.  If any node is
  * unsupported, returns CBX_ERR_UNSUPPORTED naming it and launches nothing.
- * *n_launches (may be NULL) gets the number of kernel launches issued.    */
+ * *n_launches (may be NULL) gets the number of planned launches run.  They
+ * are issued as fewer kernels where several can share one (independent
+ * element-wise launches or softmaxes, chains of row launches, ResBlock
+ * layers): the kept tensors are those of the launches in their order, a
+ * ResBlock layer's first conv output that nothing else reads and keep does
+ * not name may stay unstored.                                              */
 int cbx_graph_compute(const cbx_tensor* tensors, int32_t n_tensors,
                       const cbx_gnode* nodes, int32_t n_nodes,
                       const int32_t* keep, int32_t n_keep,
@@ -799,8 +804,8 @@ int cbx_graph_compute(const cbx_tensor* tensors, int32_t n_tensors,
  * whatever the launch count) over whatever the buffers hold then.  A
  * change of address, shape or parameter needs cbx_graph_exec_update.  Launch on the
  * device current at creation.  Unsupported nodes: CBX_ERR_UNSUPPORTED as in
- * cbx_graph_compute.  *n_launches (may be NULL) gets the kernel launch
- * count of one replay.  Each exec holds a HIP stream of its own, which its
+ * cbx_graph_compute.  *n_launches (may be NULL) gets the count of planned
+ * launches of one replay (issued as in cbx_graph_compute).  Each exec holds a HIP stream of its own, which its
  * captures are recorded on (nothing runs on it), and two instantiations of
  * the graph, which take turns (cbx_graph_exec_update), until it is
  * destroyed.  Destroy waits for the exec's own replays (not for other work
@@ -817,8 +822,8 @@ void cbx_graph_exec_destroy(cbx_graph_exec* exec);
  * loop: t3.cpp:604's decode graph with the position and the KV views of the
  * next token).  The list is planned and recorded again; when it gives the
  * same launches with other arguments (addresses, shapes, positions), the
- * instantiated graph takes them in place (*in_place = 1), otherwise it is
- * re-instantiated (*in_place = 0).  Stream-ordered: the exec's two
+ * instantiated graph takes them in place (*in_place = 1; a list it holds
+ * already changes nothing), otherwise it is re-instantiated (*in_place = 0).  Stream-ordered: the exec's two
  * instantiations take turns, and an update re-points the one not replayed
  * since the previous update, after waiting (on events recorded by that
  * update) for its replays -- all issued before the previous update -- and

@@ -210,6 +210,9 @@ def load() -> ctypes.CDLL:
         "cbx_graph_plan": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
                                ctypes.POINTER(ctypes.c_int32), ctypes.c_int32, ctypes.POINTER(GLaunch),
                                ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]),
+        "cbx_graph_steps": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
+                                ctypes.POINTER(ctypes.c_int32), ctypes.c_int32, ctypes.c_int32,
+                                ctypes.POINTER(ctypes.c_int32), ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]),
         "cbx_graph_launch": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
                                  ctypes.POINTER(GLaunch), vp]),
         "cbx_graph_compute": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
@@ -1051,6 +1054,22 @@ class Graph:
         _check(load().cbx_graph_plan(T, len(self._descs), N, len(self.nodes), K, len(keep), out, cap,
                                      ctypes.byref(n)))
         return [(out[k].kind, out[k].first_node, out[k].n_nodes, out[k].flags) for k in range(n.value)]
+
+    def steps(self, keep=(), n_cu: int = 0) -> list:
+        """The planned launches of each step that compute() or a replay issues
+        as one kernel, in order.  n_cu > 0: on a device of that many CUs, asked
+        without one."""
+        T, N, K = self._arrays(keep)
+        cap = max(1, len(self.nodes))
+        at = (ctypes.c_int32 * cap)()
+        n = ctypes.c_int32(0)
+        _check(load().cbx_graph_steps(T, len(self._descs), N, len(self.nodes), K, len(keep), n_cu, at, cap,
+                                      ctypes.byref(n)))
+        out = [[] for _ in range(max(at[:n.value], default=-1) + 1)]
+        for i, s in enumerate(at[:n.value]):
+            if s >= 0:
+                out[s].append(i)
+        return out
 
     def compute(self, keep=()) -> int:
         """Runs the nodes (cbx_graph_compute); returns the number of launches."""

@@ -215,6 +215,7 @@ int cbx_init(int device) {
     }
     DeviceState& st = g_dev[device];
     if (st.ready) return CBX_OK;
+    st.device = device;
     int prev = 0;
     hipGetDevice(&prev);
     if (hipSetDevice(device) != hipSuccess) return set_error(CBX_ERR_HIP, "cbx_init: hipSetDevice failed");
@@ -1076,7 +1077,7 @@ void cbx_conv1d_weights_destroy(cbx_conv1d_weights* w) {
 // Checks shared by cbx_conv1d and cbx_conv_transpose1d: the handle's device
 // and kind, x against the weights, y's shape (t_out), bias, res, the snake
 // vectors, and that y does not overlap x.  Sets *empty for an empty y.
-static int check_conv_io(const char* what, const cbx_conv1d_weights* w, bool transposed, int prologue,
+static int check_conv_io(const char* what, const cbx_conv1d_weights* w, int device, bool transposed, int prologue,
                          const cbx_tensor* x, const cbx_tensor* alpha, const cbx_tensor* alpha_inv,
                          const cbx_tensor* bias, const cbx_tensor* res, const cbx_tensor* y, int64_t t_out,
                          const char* t_out_rule, bool* empty) {
@@ -1087,10 +1088,7 @@ static int check_conv_io(const char* what, const cbx_conv1d_weights* w, bool tra
         return set_error(CBX_ERR_INVALID_ARG, f + (transposed ? ": the weights were made for cbx_conv1d"
                                                               : ": the weights were made for cbx_conv_transpose1d"));
     }
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev != w->device) {
-        return set_error(CBX_ERR_INVALID_ARG, f + ": the weights belong to another device");
-    }
+    if (device != w->device) return set_error(CBX_ERR_INVALID_ARG, f + ": the weights belong to another device");
     if (y->type != CBX_TYPE_F32) return set_error(CBX_ERR_UNSUPPORTED, f + ": F32 only");
     if (y->ne[0] != w->c_out || y->ne[1] != t_out || y->ne[2] != x->ne[2] || y->ne[3] != 1) {
         return set_error(CBX_ERR_INVALID_ARG, f + ": y must be (C_out, T_out, B, 1), " + t_out_rule);
@@ -1154,12 +1152,11 @@ static int check_conv_x(const char* what, const cbx_conv1d_weights* w, const cbx
 
 extern "C++" {
 
-// Everything a cbx_conv1d / cbx_conv1d_sum call checks before it launches.
-static int check_conv1d(const char* what, const ConvCall& c, DeviceState** st, bool* empty) {
+// Everything a cbx_conv1d / cbx_conv1d_sum call on `device` checks before it
+// launches.  Host code only.
+static int check_conv1d(const char* what, const ConvCall& c, int device, bool* empty) {
     int rc;
     *empty = false;
-    *st = current_state(&rc);
-    if (!*st) return rc;
     if (!c.w) return set_error(CBX_ERR_INVALID_ARG, std::string(what) + ": weights are NULL");
     if ((rc = validate(c.x, what, "x")) || (rc = validate(c.y, what, "y"))) return rc;
     if ((rc = check_conv_x(what, c.w, c.x, c.prologue))) return rc;
@@ -1169,7 +1166,7 @@ static int check_conv1d(const char* what, const ConvCall& c, DeviceState** st, b
     const int64_t t_in = c.x->ne[1];
     const int64_t span = c.dilation * (c.w->k - 1) + 1;
     const int64_t t_out = t_in + 2 * c.pad >= span ? (t_in + 2 * c.pad - span) / c.stride + 1 : 0;
-    if ((rc = check_conv_io(what, c.w, false, c.prologue, c.x, c.alpha, c.alpha_inv, c.bias, c.res, c.y, t_out,
+    if ((rc = check_conv_io(what, c.w, device, false, c.prologue, c.x, c.alpha, c.alpha_inv, c.bias, c.res, c.y, t_out,
                             "T_out = (T_in + 2 pad - dilation (K - 1) - 1) / stride + 1", empty))) {
         return rc;
     }
@@ -1187,9 +1184,11 @@ static int check_conv1d(const char* what, const ConvCall& c, DeviceState** st, b
 
 int cbx::conv1d_call(const ConvCall& c, cbx_stream stream) {
     clear_error();
-    DeviceState* st = nullptr;
+    int rc;
+    DeviceState* st = current_state(&rc);
+    if (!st) return rc;
     bool empty = false;
-    const int rc = check_conv1d(c.acc ? "cbx_conv1d_sum" : "cbx_conv1d", c, &st, &empty);
+    rc = check_conv1d(c.acc ? "cbx_conv1d_sum" : "cbx_conv1d", c, st->device, &empty);
     if (rc || empty) return rc;
     const bool snake = c.prologue == CBX_CONV_PRO_SNAKE;
     return launch_conv1d(c.x, c.w->data, c.w->k, c.w->c_in_pad, c.w->c_out, c.stride, c.pad, c.dilation, 1, 0, c.w->w_ph,
@@ -1201,7 +1200,7 @@ int cbx::conv1d_call(const ConvCall& c, cbx_stream stream) {
 // every vector access aligned, and no output byte shared with an input: its
 // workgroups read x's halo rows while others store y (one by one, conv2 may
 // write over its residual).
-bool cbx::res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int* ch) {
+bool cbx::res_layer_of(const ConvCall& c1, const ConvCall& c2, const DeviceState* st, ResLayer* l, int* ch) {
     if (!c1.w || !c2.w || c1.prologue != CBX_CONV_PRO_SNAKE || c2.prologue != CBX_CONV_PRO_SNAKE || c1.res || c1.acc ||
         !c1.bias || !c2.bias || !c2.res || c1.y != c2.x || c1.stride != 1 || c2.stride != 1 ||
         2 * static_cast<int64_t>(c1.pad) != (c1.w->k - 1) * c1.dilation ||
@@ -1209,9 +1208,8 @@ bool cbx::res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int*
         c2.w->c_in != c2.w->c_out || c1.w->c_in != c2.w->c_in) {
         return false;
     }
-    DeviceState* st = nullptr;
     bool e1 = false, e2 = false;
-    if (check_conv1d("cbx_conv1d", c1, &st, &e1) || check_conv1d("cbx_conv1d", c2, &st, &e2) || e1 || e2) {
+    if (check_conv1d("cbx_conv1d", c1, st->device, &e1) || check_conv1d("cbx_conv1d", c2, st->device, &e2) || e1 || e2) {
         clear_error();   // the calls report it when they run one by one
         return false;
     }
@@ -1292,7 +1290,7 @@ int cbx_conv_transpose1d(const cbx_tensor* x, const cbx_conv1d_weights* w, int p
     }
     const int64_t t_out = t_in > 0 ? full - 2 * static_cast<int64_t>(pad) : 0;
     bool empty = false;
-    if ((rc = check_conv_io(what, w, true, prologue, x, alpha, alpha_inv, bias, nullptr, y, t_out,
+    if ((rc = check_conv_io(what, w, st->device, true, prologue, x, alpha, alpha_inv, bias, nullptr, y, t_out,
                             "T_out = (T_in - 1) * stride + K - 2 pad", &empty))) {
         return rc;
     }
@@ -1323,8 +1321,8 @@ int cbx_causal_conv1d(const cbx_tensor* x, const cbx_conv1d_weights* w, const cb
         }
     }
     bool empty = false;
-    if ((rc = check_conv_io(what, w, false, CBX_CONV_PRO_NONE, x, nullptr, nullptr, bias, nullptr, y, x->ne[1],
-                            "T_out = T_in (left padding K - 1)", &empty))) {
+    if ((rc = check_conv_io(what, w, st->device, false, CBX_CONV_PRO_NONE, x, nullptr, nullptr, bias, nullptr, y,
+                            x->ne[1], "T_out = T_in (left padding K - 1)", &empty))) {
         return rc;
     }
     if (empty) return CBX_OK;

@@ -1644,7 +1644,7 @@ struct Scheduler {
         ResLayer r;
         ConvCall c1, c2;
         const bool ok = conv_call_of(t, nd, ls[i], &c1) == CBX_OK && conv_call_of(t, nd, ls[i + 1], &c2) == CBX_OK &&
-                        res_layer_of(c1, c2, &r, ch);
+                        res_layer_of(c1, c2, st, &r, ch);
         clear_error();
         return ok;
     }
@@ -1772,9 +1772,8 @@ struct Scheduler {
 };
 
 std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd, int32_t n,
-                           const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep) {
-    int rc = CBX_OK;
-    const DeviceState* st = current_state(&rc);
+                           const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep,
+                           const DeviceState* st) {
     if (!st) {   // the launches report it
         std::vector<Step> one;
         for (size_t i = 0; i < ls.size(); i++) {
@@ -1793,6 +1792,12 @@ std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd
         }
     }
     return std::move(s.run(n_t));
+}
+
+std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd, int32_t n,
+                           const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep) {
+    int rc = CBX_OK;
+    return schedule(t, n_t, nd, n, ls, keep, n_keep, current_state(&rc));
 }
 
 // A chain's links as the kernel takes them, each operand from memory or
@@ -1835,7 +1840,7 @@ int run_step(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const st
             for (int32_t m = 0; m < st.n; m += 2) {
                 ConvCall c1, c2;
                 if (conv_call_of(t, nd, L(m), &c1) || conv_call_of(t, nd, L(m + 1), &c2) ||
-                    !res_layer_of(c1, c2, &r[m / 2], &ch)) {
+                    !res_layer_of(c1, c2, ds, &r[m / 2], &ch)) {
                     return changed();
                 }
             }
@@ -1906,6 +1911,29 @@ int cbx_graph_plan(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gnode
                                                   " launches do not fit max_launches");
     }
     for (size_t k = 0; k < ls.size(); k++) launches[k] = ls[k];
+    return CBX_OK;
+}
+
+int cbx_graph_steps(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gnode* nodes, int32_t n_nodes,
+                    const int32_t* keep, int32_t n_keep, int32_t n_cu, int32_t* step, int32_t max_launches,
+                    int32_t* n_launches) {
+    clear_error();
+    std::vector<cbx_glaunch> ls;
+    int rc = plan(tensors, n_tensors, nodes, n_nodes, keep, n_keep, &ls, "cbx_graph_steps");
+    if (n_launches) *n_launches = static_cast<int32_t>(ls.size());
+    if (rc) return rc;
+    if (static_cast<int64_t>(ls.size()) > max_launches || (!step && !ls.empty())) {
+        return set_error(CBX_ERR_INVALID_ARG, "cbx_graph_steps: the launches do not fit max_launches");
+    }
+    DeviceState host;
+    const DeviceState* st = &host;
+    if (n_cu > 0) host.n_cu = n_cu;
+    else if (!(st = current_state(&rc))) return rc;
+    std::fill(step, step + ls.size(), -1);
+    const std::vector<Step> steps = schedule(tensors, n_tensors, nodes, n_nodes, ls, keep, n_keep, st);
+    for (size_t i = 0; i < steps.size(); i++) {
+        for (int32_t m = 0; m < steps[i].n; m++) step[steps[i].li[m]] = static_cast<int32_t>(i);
+    }
     return CBX_OK;
 }
 

@@ -48,6 +48,7 @@ inline View null_view() {
 // Per-device state created by cbx_init.
 struct DeviceState {
     bool      ready = false;
+    int       device = -1;
     int       n_cu = 0;
     uint16_t* gelu_table = nullptr;   // 65536 fp16 codes
     uint32_t* err_word = nullptr;     // sticky device error bits
@@ -195,7 +196,7 @@ struct ConvCall {
 int conv1d_call(const ConvCall& c, cbx_stream stream);
 // Whether c1 then c2 are a ResBlock layer (c2 reads c1's output, which the
 // caller says nothing else reads) that one launch takes: *l is filled.
-bool res_layer_of(const ConvCall& c1, const ConvCall& c2, ResLayer* l, int* ch);
+bool res_layer_of(const ConvCall& c1, const ConvCall& c2, const DeviceState* st, ResLayer* l, int* ch);
 // ---- several launches of a node list in one kernel (k_group.hip) ------------
 // y = act((x op b) + b2) over n4 float4s, contiguous, 16-byte aligned.
 // How b runs against x: along its rows, a value a row (rows of whole float4s,
@@ -360,3 +361,11 @@ enum { NORM_LN = 0, NORM_RMS = 1 };
 enum { UNARY_LEAKY = 100 };
 
 }  // namespace cbx
+
+// For tests and tools: the step (what a compute or a replay issues as one
+// kernel, in order) of each planned launch, -1 for a view.  n_cu > 0 asks for
+// a device of that many CUs (device -1 in the weights' handles) without one;
+// 0 for the current device.
+extern "C" int cbx_graph_steps(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gnode* nodes, int32_t n_nodes,
+                               const int32_t* keep, int32_t n_keep, int32_t n_cu, int32_t* step, int32_t max_launches,
+                               int32_t* n_launches);

@@ -1604,13 +1604,14 @@ struct Scheduler {
 
     // Adds what a launch reads and stores to rd and wr: its nodes' operands
     // and results, less the intermediates that only its own nodes read and
-    // nothing keeps (never stored).  A view stands for its source.
-    void accesses(const cbx_glaunch& l) {
+    // nothing keeps (never stored) and reads of tensor `skip`.  A view stands
+    // for its source.
+    void accesses(const cbx_glaunch& l, int32_t skip = -1) {
         const int32_t a = l.first_node, z = l.first_node + l.n_nodes;
         for (int32_t i = a; i < z; i++) {
             if (nd[i].op != CBX_GOP_VIEW && !inner(l, nd[i].dst, i)) touch(&wr, nd[i].dst);
             for (int32_t s : nd[i].src) {
-                if (s < 0) continue;
+                if (s < 0 || s == skip) continue;
                 bool made = false;   // by a node of the launch
                 for (int32_t j = a; j < i; j++) made = made || nd[j].dst == s;
                 if (!made) touch(&rd, s);
@@ -1707,11 +1708,10 @@ struct Scheduler {
                 s.kind = kStepLayers;
                 s.li[s.n++] = static_cast<int32_t>(i);
                 f.key = ch;
-                // conv1's output is neither stored nor read
-                const int32_t h = cls[static_cast<size_t>(nd[l.first_node + l.n_nodes - 1].dst)];
+                // conv1's output is neither stored nor read (that tensor: what
+                // else its bytes' class holds, x or the residual, is read)
                 wr.clear();
-                accesses(ls[i++]);
-                rd.erase(std::remove(rd.begin(), rd.end(), h), rd.end());
+                accesses(ls[i++], nd[l.first_node + l.n_nodes - 1].dst);
             } else if (l.kind == CBX_GL_CONCAT) {
                 while (s.n < kConcatMax && appends(i)) s.li[s.n++] = static_cast<int32_t>(i++);
                 // the longest run of them that is plain copies

@@ -57,3 +57,59 @@ def test_refuses_a_short_array():
     n = C.ctypes.c_int32(0)
     assert C.load().cbx_graph_steps(T, 2, N, 1, None, 0, 64, None, 0, C.ctypes.byref(n)) == C.ERR_INVALID_ARG
     assert n.value == 1
+
+
+# ---- buffers used again -----------------------------------------------------------
+
+def step_of(l, keep, i):
+    """The step whose launches make tensor i."""
+    plan = l.g.plan(keep)
+    for s, launches in enumerate(l.steps(keep)):
+        if any(l.g.nodes[plan[k][1] + plan[k][2] - 1].dst == i for k in launches):
+            return s
+    raise AssertionError(i)
+
+
+@pytest.mark.parametrize("bridge", ["x", "residual only"])
+def test_layer_after_the_one_it_reads(bridge):
+    """Layer 2 reads layer 1's result y1. Its first conv's output lies in the
+    same arena, and an earlier tensor spans both: the class of bytes that the
+    never-stored output is in holds y1 as well."""
+    ch, T = 64, 12000
+    n = ch * T
+    l = HostList()
+    arena = torch.empty(3 * n + 64)
+    span = l.t(arena[:2 * n].view(2 * T, ch))
+    dead = l.scale(span, 2.0)                                  # reads the arena before it is used again
+    y1, _ = l.layer(l.x(T, ch), ch, 3, 1)
+    if bridge == "x":
+        l.place(y1, arena, 0)
+        y2, h2 = l.layer(y1, ch, 3, 3)
+    else:                                                      # x of its own, the residual is y1
+        x2 = l.x(T, ch)
+        y2, h2 = l.layer(x2, ch, 3, 3)
+        l.place(y1, arena, 0)
+        add = l.g.nodes[-1]
+        add.src[0] = y1
+    l.place(h2, arena, n)
+    keep = [dead, y1, y2]
+    assert step_of(l, keep, y1) < step_of(l, keep, y2)
+
+
+def test_write_over_what_a_layer_reads():
+    """A launch after the layer that writes over its input stays after it,
+    also when an earlier step of its kind has room."""
+    ch, T = 64, 12000
+    n = ch * T
+    l = HostList()
+    arena = torch.empty(2 * n + 64)
+    span = l.t(arena[:2 * n].view(2 * T, ch))
+    early = l.scale(l.x(T, ch), 2.0)                           # an element-wise step ahead of the layer
+    x = l.t(arena[:n].view(T, ch))
+    y, h = l.layer(x, ch, 3, 1)
+    l.place(h, arena, n)
+    over = l.scale(l.x(T, ch), 3.0)                            # over x
+    l.place(over, arena, 0)
+    keep = [early, y, over]
+    assert span >= 0 and step_of(l, keep, early) < step_of(l, keep, over)
+    assert step_of(l, keep, y) < step_of(l, keep, over)

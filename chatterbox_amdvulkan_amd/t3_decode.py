@@ -147,21 +147,35 @@ class T3DecodeStep:
         """The list of the token after n_past cached ones: the score views
         (n_past + 1 columns a head, same first element) and the mask's n_past
         change; the graph's tensor indices and launches stay the same.  The
-        descriptors are patched in place (the graph's arrays are bound)."""
+        list's descriptors and nodes are set in place."""
         if not 0 <= n_past < self.max_ctx:
             raise ValueError(f"n_past {n_past} outside [0, {self.max_ctx})")
         n_kv = n_past + 1
-        t, n = self._arrays()
-        ids = self._score_ids
-        t["ne"][ids, 0] = n_kv
-        t["nb"][ids, 1:3] = 4 * n_kv
-        t["nb"][ids, 3] = 4 * n_kv * self.n_head
-        n["iparam"][self._mask_nodes] = n_past
+        ids, plane = self._score_ids, 4 * n_kv * self.n_head
+        bound = self._bound_arrays()
+        if bound is not None:
+            t, n = bound
+            t["ne"][ids, 0] = n_kv
+            t["nb"][ids, 1:3] = 4 * n_kv
+            t["nb"][ids, 3] = plane
+            n["iparam"][self._mask_nodes] = n_past
+        else:                       # a node or tensor was added: one by one
+            for i in ids:
+                d = self.graph._descs[i]
+                d.ne[0] = n_kv
+                d.nb[1] = d.nb[2] = 4 * n_kv
+                d.nb[3] = plane
+            for k in self._mask_nodes:
+                self.graph.nodes[k].iparam = n_past
         self.n_past = n_past
 
-    def _arrays(self):
-        """The bound descriptor and node arrays as numpy records."""
-        T, N, _ = self.graph._arrays(self.keep)
+    def _bound_arrays(self):
+        """The arrays that the graph's descriptors and nodes are views of, as
+        numpy records, under whatever keep list they were bound; None when
+        they are bound to none."""
+        if self.graph._bound is None:
+            return None
+        T, N = self.graph._bound[:2]
         if self._views is None or self._views[0] is not T:
             self._views = (T, np.frombuffer(T, TENSOR_FIELDS), np.frombuffer(N, NODE_FIELDS))
         return self._views[1:]

@@ -6,8 +6,11 @@ the operands the reference's builder gives them.  Planting a wrong operand
 parameters of the wrong block, the mask without n_past) fails it."""
 import numpy as np
 import pytest
+import torch
 
+from chatterbox_amdvulkan_amd import cbxops as C
 from chatterbox_amdvulkan_amd import workloads as W
+from chatterbox_amdvulkan_amd.t3_decode import T3DecodeStep
 from tests._util import assert_bitexact
 
 H = W.T3_HEADS
@@ -64,3 +67,27 @@ def test_scores_mask_nothing_at_n_kv(oracle):
     assert p.shape == (H, 41)
     assert (p > 0).all()
     np.testing.assert_allclose(p.sum(axis=1), 1.0, rtol=1e-6)
+
+
+@pytest.mark.parametrize("how", ["bound", "another keep list", "a node added", "bound under another keep"])
+def test_retarget_reaches_the_list(how):
+    """retarget() changes the list itself, whatever arrays it is bound to: the
+    next update or compute passes the new lengths and mask."""
+    dev = {k: torch.from_numpy(v) for k, v in small_inputs(L=2).items()}
+    dev["token"] = dev["position"] = torch.zeros(1, dtype=torch.int32)
+    st = T3DecodeStep(dev, 3)
+    if how == "another keep list":
+        st.keep = st.keep + [st.keep[0]]
+    elif how == "a node added":
+        y = st.graph.tensor(torch.zeros(1, W.D_MODEL))
+        st.graph.node(C.GOP_SCALE, y, (st.keep[-1],), fparam=2.0)
+    elif how == "bound under another keep":
+        st.graph.bind_arrays(st.keep[:-1])
+    for n_past in (9, 4):
+        st.retarget(n_past)
+        T, N, _ = st.graph._arrays(st.keep)
+        for ids in st._kq_ids:
+            for i in ids:
+                assert list(T[i].ne) == [n_past + 1, 1, H, 1]
+                assert list(T[i].nb) == [4, 4 * (n_past + 1), 4 * (n_past + 1), 4 * (n_past + 1) * H]
+        assert [N[k].iparam for k in st._mask_nodes] == [n_past] * 2

@@ -1317,6 +1317,7 @@ int elt_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, EltOp
             const cbx_tensor *b = T(t, a.src[1]), *V = T(t, v.dst);
             if (v.op != CBX_GOP_VIEW || !b || !V || !row_of(b, x->ne[0])) return 0;
             int n = 0;
+            const cbx_tensor *vecs[2], *outs[2];
             for (int32_t k = f + 2; k < f + l.n_nodes; k++) {
                 const cbx_gnode& g = nd[k];
                 if (g.op == CBX_GOP_VIEW) continue;
@@ -1337,9 +1338,16 @@ int elt_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, EltOp
                 if (bytes_overlap(o, u) || bytes_overlap(o, x) || !elt_binary(x, b, &oy, e + n)) return 0;
                 e[n].b2 = static_cast<const float*>(u->data);
                 e[n].C2 = static_cast<uint32_t>(nelements(u));
+                vecs[n] = u;
+                outs[n] = o;
                 n++;
             }
-            if (n != 2) return 0;
+            // the two run side by side: as cbx_bias_add_pair refuses it,
+            // neither output meets the other or the other's vector
+            if (n != 2 || bytes_overlap(outs[0], outs[1]) || bytes_overlap(outs[0], vecs[1]) ||
+                bytes_overlap(outs[1], vecs[0])) {
+                return 0;
+            }
             return n;
         }
         case CBX_GL_UNARY:

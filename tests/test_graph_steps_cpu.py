@@ -113,3 +113,37 @@ def test_write_over_what_a_layer_reads():
     keep = [early, y, over]
     assert span >= 0 and step_of(l, keep, early) < step_of(l, keep, over)
     assert step_of(l, keep, y) < step_of(l, keep, over)
+
+
+# ---- what an entry point refuses runs alone, where it is refused ----------------------
+
+def bias_pair(l, T=64, D=512, heads=8):
+    """add(x, bias) -> heads view -> add(., u), add(., v); the tensors by name."""
+    t = {"x": l.x(T, D), "bias": l.x(D), "u": l.x(heads, D // heads), "v": l.x(heads, D // heads)}
+    s = l.add(t["x"], t["bias"])
+    w = l.node_view(l.at(s).view(T, heads, D // heads), s)
+    t["yu"], t["yv"] = l.add(w, t["u"]), l.add(w, t["v"])
+    return t
+
+
+@pytest.mark.parametrize("out,over", [(None, None), ("yu", "yv"), ("yu", "v"), ("yv", "u"), ("yu", "u"), ("yv", "v"),
+                                      ("yu", "bias"), ("yv", "x")])
+def test_bias_pair_over_its_own_tensors(out, over):
+    """cbx_bias_add_pair refuses an output over an input or the other output:
+    such a launch joins no group (alone, it is refused)."""
+    l = HostList()
+    other = l.add(l.x(64, 512), l.x(512))
+    l.scale(other, 2.0)
+    t = bias_pair(l)
+    if out:
+        n = max(l.at(t[out]).numel(), l.at(t[over]).numel())
+        buf = torch.empty(n + 64)
+        # the graph's descriptors follow the tensors: views of x and the sum keep theirs
+        for k in (out, over):
+            l.place(t[k], buf, 0)
+    keep = [other, t["yu"], t["yv"]]
+    plan = l.g.plan(keep)
+    pair = [i for i, p in enumerate(plan) if p[0] == C.GL_BIAS_ADD_PAIR]
+    assert len(pair) == 1
+    step, = [s for s in l.steps(keep) if pair[0] in s]
+    assert (len(step) == 1) == bool(out)

@@ -1248,8 +1248,14 @@ struct Step {
     bool operator==(const Step& o) const { return kind == o.kind && n == o.n && std::equal(li, li + n, o.li); }
 };
 
+// A descriptor the entry points take (validate()'s terms): what they refuse
+// runs alone, where they refuse it.
+bool sound(const cbx_tensor* t) {
+    return t && t->data && t->reserved == 0 && t->ne[0] >= 0 && t->ne[1] >= 0 && t->ne[2] >= 0 && t->ne[3] >= 0;
+}
+
 bool f32_flat16(const cbx_tensor* t) {
-    return t && t->data && t->type == CBX_TYPE_F32 && is_contiguous(t) && reinterpret_cast<uintptr_t>(t->data) % 16 == 0;
+    return sound(t) && t->type == CBX_TYPE_F32 && is_contiguous(t) && reinterpret_cast<uintptr_t>(t->data) % 16 == 0;
 }
 
 // t is one row of n floats
@@ -1270,7 +1276,7 @@ bool elt_binary(const cbx_tensor* x, const cbx_tensor* b, const cbx_tensor* y, E
     e->ne0_4 = static_cast<uint32_t>(x->ne[0] / 4);
     e->act = CBX_UNARY_NONE;
     if (!b) return true;
-    if (b->type != CBX_TYPE_F32 || !b->data || !is_contiguous(b) || bytes_overlap(b, y)) return false;
+    if (!sound(b) || b->type != CBX_TYPE_F32 || !is_contiguous(b) || bytes_overlap(b, y)) return false;
     e->b = static_cast<const float*>(b->data);
     if (rows4 && row_of(b, x->ne[0])) {
         e->bmode = kEltVec;
@@ -1315,7 +1321,7 @@ int elt_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, EltOp
             // add(x, bias) -> heads view -> [views] add(view, u), add(view, v)
             const cbx_gnode& v = nd[f + 1];
             const cbx_tensor *b = T(t, a.src[1]), *V = T(t, v.dst);
-            if (v.op != CBX_GOP_VIEW || !b || !V || !row_of(b, x->ne[0])) return 0;
+            if (v.op != CBX_GOP_VIEW || !b || !sound(V) || !row_of(b, x->ne[0])) return 0;
             int n = 0;
             const cbx_tensor *vecs[2], *outs[2];
             for (int32_t k = f + 2; k < f + l.n_nodes; k++) {
@@ -1375,8 +1381,9 @@ int elt_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, EltOp
 }
 
 // The copies of concats along dim 0 at planned launches li[0 .. n), each
-// appending to the one before it (whose result only it reads): one per
-// source, into the last one's result.  The count (n + 1), or 0.
+// appending to the one before it (whose result only it reads, and which
+// cbx_concat would take): one per source, into the last one's result.  The
+// count (n + 1), or 0.
 constexpr int kConcatMax = 4;
 int concat_of(const cbx_tensor* t, const cbx_gnode* nd, const std::vector<cbx_glaunch>& ls, const int32_t* li, int32_t n,
               EltOp* e) {
@@ -1404,8 +1411,17 @@ int concat_of(const cbx_tensor* t, const cbx_gnode* nd, const std::vector<cbx_gl
             off += x->ne[0];
             k++;
         }
+        // the result so far, stored or not
+        const cbx_tensor* r = T(t, g.dst);
+        if (!sound(r) || r->type != CBX_TYPE_F32 || r->nb[0] != sizeof(float) || r->ne[0] != off ||
+            r->ne[1] != y->ne[1] || r->ne[2] != y->ne[2] || r->ne[3] != y->ne[3]) {
+            return 0;
+        }
+        for (int32_t s : g.src) {
+            if (bytes_overlap(r, &t[s])) return 0;
+        }
     }
-    return off == y->ne[0] ? k : 0;
+    return k;
 }
 
 // A planned softmax as a call (run()'s reading of it), its group key >= 0.
@@ -1424,7 +1440,7 @@ bool softmax_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, 
         else return false;
     }
     for (const cbx_tensor* p : {c->x, add ? c->b : c->x, static_cast<const cbx_tensor*>(c->y)}) {
-        if (!p || !p->data || p->type != CBX_TYPE_F32 || p->nb[0] != sizeof(float) || !same_shape(p, c->x) ||
+        if (!sound(p) || p->type != CBX_TYPE_F32 || p->nb[0] != sizeof(float) || !same_shape(p, c->x) ||
             nelements(p) == 0) {
             return false;
         }
@@ -1517,7 +1533,7 @@ bool link_of(const cbx_tensor* t, const cbx_gnode* nd, const cbx_glaunch& l, Lin
         default: return false;
     }
     if (!k->a || !out) return false;
-    if (k->mask && (k->mask->type != CBX_TYPE_F32 || !k->mask->data || !is_contiguous(k->mask) || k->mask->ne[0] != 1 ||
+    if (k->mask && (!sound(k->mask) || k->mask->type != CBX_TYPE_F32 || !is_contiguous(k->mask) || k->mask->ne[0] != 1 ||
                     k->mask->ne[1] != k->a->ne[1] || nelements(k->mask) != nrows(k->a))) {
         return false;
     }

@@ -147,3 +147,62 @@ def test_bias_pair_over_its_own_tensors(out, over):
     assert len(pair) == 1
     step, = [s for s in l.steps(keep) if pair[0] in s]
     assert (len(step) == 1) == bool(out)
+
+
+def grouped(l, keep, dst):
+    """Whether the launch making tensor dst shares its step."""
+    plan = l.g.plan(keep)
+    k, = [i for i, p in enumerate(plan) if l.g.nodes[p[1] + p[2] - 1].dst == dst]
+    step, = [s for s in l.steps(keep) if k in s]
+    return len(step) > 1
+
+
+@pytest.mark.parametrize("form", ["add", "bias", "mask", "unary", "scale", "soft_max", "rows", "rows w", "concat"])
+def test_descriptor_no_entry_point_takes(form):
+    """A descriptor that every entry point refuses (reserved set) does not pass
+    in a group's name."""
+    l = HostList()
+    T, D = 64, 256
+    a = l.x(T, D)
+    if form in ("add", "bias", "mask", "unary", "scale"):
+        bad = l.x(*{"bias": (D,), "mask": (T, 1)}.get(form, (T, D)))
+        first = l.scale(l.x(T, D), 2.0)
+        y = (l.unary(bad, C.TANH) if form == "unary" else l.scale(bad, 2.0) if form == "scale"
+             else l.mul(a, bad) if form == "mask" else l.add(a, bad))
+    elif form == "soft_max":
+        bad = l.x(8, T, T)
+        first, y = l.soft_max(l.x(8, T, T)), l.soft_max(bad)
+    elif form == "concat":
+        bad = l.x(T, 80)
+        first = l.concat(l.x(T, 80), bad, 0)
+        y = l.concat(first, l.x(T, 80), 0)
+    else:
+        w = l.x(D)
+        first = l.layer_norm(l.add(a, l.x(T, D)), l.x(D), l.x(D))
+        bad = w if form == "rows w" else l.x(T, D)
+        y = l.layer_norm(l.add(first, bad if form == "rows" else l.x(T, D)), w, l.x(D))
+    keep = [y] if form == "concat" else [first, y]
+    assert grouped(l, keep, y)
+    l.g._descs[bad].reserved = 1
+    assert not grouped(l, keep, y)
+
+
+@pytest.mark.parametrize("what", ["type", "rows", "columns", "over a source"])
+def test_concat_run_with_a_bad_intermediate(what):
+    """cbx_concat would refuse the intermediate result: the concats run one by one."""
+    l = HostList()
+    T = 32
+    srcs = [l.x(T, 80) for _ in range(3)]
+    a = l.concat(srcs[0], srcs[1], 0)
+    y = l.concat(a, srcs[2], 0)
+    assert grouped(l, [y], y)
+    d = l.g._descs[a]
+    if what == "type":
+        d.type = C.F16
+    elif what == "rows":
+        d.ne[1] = T + 1
+    elif what == "columns":
+        d.ne[0] = 176
+    else:
+        d.data = l.at(srcs[1]).data_ptr()
+    assert not grouped(l, [y], y)

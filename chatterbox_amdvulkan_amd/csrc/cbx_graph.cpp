@@ -1595,6 +1595,7 @@ struct Scheduler {
     // the last step that reads and that writes a class is all a launch has
     // to look at.
     std::vector<int32_t> cls;                   // by tensor; -1: no bytes
+    std::vector<int32_t> order, first;          // the tensors class by class; each class's first in it
     std::vector<int32_t> last_rd, last_wr;      // by class: the last step, or -1
     std::vector<int32_t> rd, wr;                // the current launch's classes
 
@@ -1609,14 +1610,18 @@ struct Scheduler {
         std::sort(v.begin(), v.end(), [](const auto& x, const auto& y) { return x.first.lo < y.first.lo; });
         int32_t n = -1;
         uintptr_t hi = 0;
+        order.reserve(v.size());
         for (const auto& q : v) {
             if (n < 0 || q.first.lo >= hi) {
                 n++;
                 hi = 0;
+                first.push_back(static_cast<int32_t>(order.size()));
             }
             hi = std::max(hi, q.first.hi);
             cls[static_cast<size_t>(q.second)] = n;
+            order.push_back(q.second);
         }
+        first.push_back(static_cast<int32_t>(order.size()));
         last_rd.assign(static_cast<size_t>(n + 1), -1);
         last_wr.assign(static_cast<size_t>(n + 1), -1);
     }
@@ -1626,21 +1631,67 @@ struct Scheduler {
         if (c >= 0) v->push_back(c);
     }
 
-    // Adds what a launch reads and stores to rd and wr: its nodes' operands
-    // and results, less the intermediates that only its own nodes read and
-    // nothing keeps (never stored) and reads of tensor `skip`.  A view stands
-    // for its source.
-    void accesses(const cbx_glaunch& l, int32_t skip = -1) {
+    // Calls read(tensor) and write(tensor) for what a launch reads and stores:
+    // its nodes' operands and results, less the intermediates that only its
+    // own nodes read and nothing keeps (never stored).  A view stands for its
+    // source.
+    template <typename R, typename W>
+    void each_access(const cbx_glaunch& l, R read, W write) const {
         const int32_t a = l.first_node, z = l.first_node + l.n_nodes;
         for (int32_t i = a; i < z; i++) {
-            if (nd[i].op != CBX_GOP_VIEW && !inner(l, nd[i].dst, i)) touch(&wr, nd[i].dst);
+            if (nd[i].op != CBX_GOP_VIEW && !inner(l, nd[i].dst, i)) write(nd[i].dst);
             for (int32_t s : nd[i].src) {
-                if (s < 0 || s == skip) continue;
+                if (s < 0) continue;
                 bool made = false;   // by a node of the launch
                 for (int32_t j = a; j < i; j++) made = made || nd[j].dst == s;
-                if (!made) touch(&rd, s);
+                if (!made) read(s);
             }
         }
+    }
+
+    // Adds the classes that a launch reads (but for tensor `skip`) and stores
+    // to rd and wr.
+    void accesses(const cbx_glaunch& l, int32_t skip = -1) {
+        each_access(l, [&](int32_t s) { if (s != skip) touch(&rd, s); }, [&](int32_t d) { touch(&wr, d); });
+    }
+
+    // Whether tensor d's bytes, as stored before planned launch `from`, are
+    // read under another descriptor by that launch or a later one, or kept
+    // under one, before a launch stores over them: d has to be stored then.
+    bool shown(int32_t d, size_t from) const {
+        const int32_t c = cls[static_cast<size_t>(d)];
+        if (c < 0) return false;
+        const int32_t *m = order.data() + first[static_cast<size_t>(c)], *end = order.data() + first[static_cast<size_t>(c) + 1];
+        if (end - m == 1) return false;   // no other descriptor's bytes meet d's
+        std::vector<Span> live{span_of(t[d])};
+        auto meets = [&](int32_t q) {
+            if (q == d || cls[static_cast<size_t>(q)] != c) return false;
+            const Span p = span_of(t[q]);
+            for (const Span& b : live) {
+                if (p.lo < b.hi && b.lo < p.hi) return true;
+            }
+            return false;
+        };
+        bool seen = false;
+        for (size_t i = from; i < ls.size() && !live.empty(); i++) {
+            if (ls[i].kind == CBX_GL_VIEW) continue;
+            each_access(ls[i], [&](int32_t s) { seen = seen || meets(s); }, [](int32_t) {});
+            if (seen) return true;
+            each_access(ls[i], [](int32_t) {}, [&](int32_t w) {
+                if (!meets(w) || !is_contiguous(&t[w])) return;
+                const Span p = span_of(t[w]);
+                std::vector<Span> left;
+                for (const Span& b : live) {
+                    if (p.lo > b.lo) left.push_back({b.lo, std::min(b.hi, p.lo)});
+                    if (p.hi < b.hi) left.push_back({std::max(b.lo, p.hi), b.hi});
+                }
+                live.swap(left);
+            });
+        }
+        for (; m != end; m++) {
+            if (keep[static_cast<size_t>(*m)] && meets(*m)) return true;
+        }
+        return false;
     }
 
     // tensor d, made by node i of launch l, stays unstored: a later node of
@@ -1671,7 +1722,7 @@ struct Scheduler {
         const bool ok = conv_call_of(t, nd, ls[i], &c1) == CBX_OK && conv_call_of(t, nd, ls[i + 1], &c2) == CBX_OK &&
                         res_layer_of(c1, c2, st, &r, ch);
         clear_error();
-        return ok;
+        return ok && !shown(h, i + 1);
     }
 
     // Link k may follow the chain that is step `at`: the rows match, what it
@@ -1709,7 +1760,7 @@ struct Scheduler {
         if (i >= ls.size() || ls[i].kind != CBX_GL_CONCAT || ls[i - 1].kind != CBX_GL_CONCAT) return false;
         const int32_t d = nd[ls[i - 1].first_node].dst;
         return nd[ls[i].first_node].src[0] == d && nd[ls[i].first_node].src[1] != d &&
-               uses[static_cast<size_t>(d)] == 1 && !keep[static_cast<size_t>(d)];
+               uses[static_cast<size_t>(d)] == 1 && !keep[static_cast<size_t>(d)] && !shown(d, i);
     }
 
     std::vector<Step>& run(int32_t n_t) {
@@ -1808,7 +1859,7 @@ std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd
         return one;
     }
     Scheduler s{t, nd, ls, st, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
-                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}};
+                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}, {}, {}};
     for (int32_t k = 0; k < n_keep; k++) s.keep[static_cast<size_t>(keep[k])] = 1;
     for (int32_t i = 0; i < n; i++) {
         for (int32_t q : nd[i].src) {

@@ -206,3 +206,52 @@ def test_concat_run_with_a_bad_intermediate(what):
     else:
         d.data = l.at(srcs[1]).data_ptr()
     assert not grouped(l, [y], y)
+
+
+# ---- results left unstored ------------------------------------------------------------
+
+def alias(l, i):
+    """Tensor i's bytes under another descriptor, with no VIEW node."""
+    return l.t(l.at(i))
+
+
+@pytest.mark.parametrize("read", ["by a launch", "kept", "part of it", "after a write over it", "before it is made"])
+def test_layer_whose_first_output_is_read_under_another_name(read):
+    """conv1's output stays unstored only where no other descriptor of its
+    bytes shows it: one that a later launch reads, or the caller keeps."""
+    l = HostList()
+    ch, T = 64, 12000
+    x = l.x(T, ch)
+    if read == "before it is made":
+        buf = l.empty((T, ch))
+        old = l.scale(l.t(buf), 2.0)
+        y, h = l.layer(x, ch, 3, 1)
+        l.g.rebind(h, buf)
+        keep = [old, y]
+    else:
+        y, h = l.layer(x, ch, 3, 1)
+        h2 = alias(l, h) if read != "part of it" else l.t(l.at(h).view(-1)[64:64 + 640].view(10, 64))
+        keep = [y]
+        if read == "kept":
+            keep.append(h2)
+        else:
+            if read == "after a write over it":
+                over = l.scale(l.x(T, ch), 3.0)
+                l.g.rebind(over, l.at(h))
+            keep.append(l.scale(h2, 2.0))
+    fused = [s for s in kinds(l.g, keep) if s == [C.GL_CONV1D, C.GL_CONV1D]]
+    assert len(fused) == (1 if read in ("after a write over it", "before it is made") else 0)
+
+
+@pytest.mark.parametrize("read", [None, "by a launch", "kept"])
+def test_concat_run_whose_middle_is_read_under_another_name(read):
+    l = HostList()
+    T = 32
+    a = l.concat(l.x(T, 80), l.x(T, 80), 0)
+    y = l.concat(a, l.x(T, 80), 0)
+    keep = [y]
+    if read == "kept":
+        keep.append(alias(l, a))
+    elif read:
+        keep.append(l.unary(alias(l, a), C.TANH))
+    assert any(s.count(C.GL_CONCAT) == 2 for s in kinds(l.g, keep)) == (read is None)

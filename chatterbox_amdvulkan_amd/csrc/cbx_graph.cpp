@@ -1598,6 +1598,8 @@ struct Scheduler {
     std::vector<int32_t> order, first;          // the tensors class by class; each class's first in it
     std::vector<int32_t> last_rd, last_wr;      // by class: the last step, or -1
     std::vector<int32_t> rd, wr;                // the current launch's classes
+    std::vector<int64_t> floats;                // by planned launch: what its element-wise ops store
+    std::vector<char> full;                     // one unactivated op of two whole operands
 
     void classes(int32_t n_t) {
         std::vector<std::pair<Span, int32_t>> v;
@@ -1765,6 +1767,8 @@ struct Scheduler {
 
     std::vector<Step>& run(int32_t n_t) {
         classes(n_t);
+        floats.assign(ls.size(), 0);
+        full.assign(ls.size(), 0);
         for (size_t i = 0; i < ls.size();) {
             const cbx_glaunch& l = ls[i];
             const size_t at = i++;
@@ -1810,18 +1814,23 @@ struct Scheduler {
                 if (link && l.kind != CBX_GL_SCALE && l.kind != CBX_GL_BINARY) s.kind = kStepRows;
                 else if ((f.elts = elt_of(t, nd, l, eo)) > 0) s.kind = kStepElt;
             }
+            for (int k = 0; k < f.elts; k++) floats[at] += int64_t{4} * eo[k].n4;
+            full[at] = f.elts == 1 && eo[0].bmode == kEltFull && eo[0].act == CBX_UNARY_NONE;
             // one past the last step this one conflicts with
             int32_t lo = -1;
             for (int32_t c : rd) lo = std::max(lo, last_wr[static_cast<size_t>(c)]);
             for (int32_t c : wr) lo = std::max(lo, std::max(last_wr[static_cast<size_t>(c)], last_rd[static_cast<size_t>(c)]));
             const size_t from = static_cast<size_t>(lo + 1);
             size_t to = steps.size();
+            // (what no number of others makes worth sharing stays where it is: in
+            // the list's order, its operands may still be in cache)
             if (link && from > 0 && steps[from - 1].kind == kStepRows && steps[from - 1].n < kStepMax &&
                 follows(from - 1, f.link)) {
                 to = from - 1;
                 info[to].link = f.link;
                 f.elts = 0;
-            } else if (s.kind == kStepLayers || s.kind == kStepElt || s.kind == kStepSoftMax) {
+            } else if (s.kind == kStepLayers || s.kind == kStepSoftMax ||
+                       (s.kind == kStepElt && floats[at] <= most(at, true))) {
                 for (size_t q = from; q < steps.size(); q++) {
                     const bool room = steps[q].n + s.n <= (s.kind == kStepLayers ? 2 * kResMax : kStepMax) &&
                                       info[q].elts + f.elts <= kEltMax;
@@ -1842,7 +1851,66 @@ struct Scheduler {
             for (int32_t c : rd) last_rd[static_cast<size_t>(c)] = std::max(last_rd[static_cast<size_t>(c)], me);
             for (int32_t c : wr) last_wr[static_cast<size_t>(c)] = std::max(last_wr[static_cast<size_t>(c)], me);
         }
+        return settled();
+    }
+
+    // The steps with those launches taken out of their step again, each into
+    // one of its own, that are the faster alone (a group's launches do not
+    // depend on each other).
+    std::vector<Step>& settled() {
+        std::vector<Step> out;
+        out.reserve(steps.size());
+        auto alone = [&](const Step& s, int32_t m, int32_t n) {
+            Step o;
+            o.kind = n > 1 ? s.kind : kStepOne;
+            for (int32_t k = 0; k < n; k++) o.li[o.n++] = s.li[m + k];
+            out.push_back(o);
+        };
+        for (size_t q = 0; q < steps.size(); q++) {
+            const Step& s = steps[q];
+            if (s.n > 1 && s.kind == kStepElt) {
+                // entries: a launch, or a run of concats (the launches whose
+                // floats are counted with their first's)
+                auto entry = [&](int32_t m) {
+                    int32_t n = 1;
+                    while (m + n < s.n && floats[static_cast<size_t>(s.li[m + n])] == 0) n++;
+                    return n;
+                };
+                int32_t entries = 0;
+                for (int32_t m = 0; m < s.n; m += entry(m)) {
+                    entries += floats[static_cast<size_t>(s.li[m])] <= most(static_cast<size_t>(s.li[m]), true);
+                }
+                const bool four = entries >= 4;
+                Step g;
+                g.kind = kStepElt;
+                for (int32_t m = 0, n; m < s.n; m += n) {
+                    n = entry(m);
+                    if (floats[static_cast<size_t>(s.li[m])] > most(static_cast<size_t>(s.li[m]), four)) {
+                        alone(s, m, n);
+                    } else {
+                        for (int32_t k = 0; k < n; k++) g.li[g.n++] = s.li[m + k];
+                    }
+                }
+                if (g.n > 0) out.push_back(g);
+            } else {
+                out.push_back(s);
+            }
+        }
+        steps.swap(out);
         return steps;
+    }
+
+    // The floats up to which element-wise launch i shares a kernel, with three
+    // others at least or fewer.  A group's kernel takes one float4 a lane where
+    // a launch of its own takes up to four, so it pays while the launches are
+    // bound by their start (2.2 us each).  Measured on 256 CUs (bias + GELU,
+    // us, alone / grouped): 2 x 2^19 floats 6.0 / 5.6, 2 x 2^20 6.9 / 8.3, 4 x
+    // 2^20 13.3 / 13.4, 8 x 2^20 25.9 / 23.3, 8 x 2^21 33.0 / 42.7, 4 x 2^23
+    // 56.8 / 81.7.  Sums of two whole tensors, three streams each, keep pace:
+    // 4 x 2^22 34.5 / 31.6, 8 x 2^22 73.0 / 59.8, 2 x 2^23 31.1 / 32.8.
+    int64_t most(size_t i, bool four) const {
+        const int64_t small = int64_t{2048} * st->n_cu;
+        return !four ? small : full[i] ? int64_t{1} << 26 : 2 * small;
     }
 };
 
@@ -1859,7 +1927,7 @@ std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd
         return one;
     }
     Scheduler s{t, nd, ls, st, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
-                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}, {}, {}};
+                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
     for (int32_t k = 0; k < n_keep; k++) s.keep[static_cast<size_t>(keep[k])] = 1;
     for (int32_t i = 0; i < n; i++) {
         for (int32_t q : nd[i].src) {

@@ -255,3 +255,69 @@ def test_concat_run_whose_middle_is_read_under_another_name(read):
     elif read:
         keep.append(l.unary(alias(l, a), C.TANH))
     assert any(s.count(C.GL_CONCAT) == 2 for s in kinds(l.g, keep)) == (read is None)
+
+
+# ---- launch sizes ----------------------------------------------------------------------
+
+class FarList(HostList):
+    """Tensors that are descriptors only: addresses of their own and no memory."""
+
+    @staticmethod
+    def empty(shape, dtype=torch.float32):
+        return torch.empty(shape, dtype=dtype, device="meta")
+
+    def steps(self, keep, n_cu=N_CU):
+        at, base = 1 << 44, {}
+        for i, t in enumerate(self.g._torch):
+            key = t.untyped_storage()._cdata
+            if key not in base:
+                base[key] = at
+                at += -(-t.untyped_storage().nbytes() // 4096) * 4096 + 4096
+            self.g._descs[i].data = base[key] + t.storage_offset() * t.element_size()
+        return super().steps(keep, n_cu)
+
+
+def test_group_of_more_work_items_than_a_grid_takes():
+    """A grid holds under 2^32 work-items, and an element-wise group takes one
+    a float4: of launches of 2^30 - 1 float4s, fewer than five share one."""
+    l = FarList()
+    keep = [l.scale(l.x((1 << 30) - 1, 4), 2.0) for _ in range(9)]
+    steps = l.steps(keep)
+    assert sum(len(s) for s in steps) == 9
+    assert all(len(s) * (1 << 30) < 1 << 32 for s in steps)
+
+
+@pytest.mark.parametrize("n,lg,shared", [(2, 19, 2), (2, 20, 0), (3, 20, 0), (4, 20, 4), (8, 20, 8), (8, 21, 0)])
+def test_group_only_where_it_is_the_faster(n, lg, shared):
+    """2^11 floats a launch and CU, twice that where four share it."""
+    l = FarList()
+    keep = [l.unary(l.add(l.x(1 << (lg - 10), 1024), l.x(1024)), C.GELU) for _ in range(n)]
+    keep += [l.unary(l.add(l.x(1 << 14, 1024), l.x(1024)), C.GELU)]            # never
+    steps = l.steps(keep)
+    assert sum(len(s) for s in steps) == n + 1 and max(len(s) for s in steps) == max(shared, 1)
+    assert [n] in steps
+
+
+def test_group_of_whole_sums_and_concat_runs():
+    """Four large sums of two whole tensors share a launch, two do not; a run
+    of concats stays one launch whatever its size."""
+    l = FarList()
+    assert len(l.steps([l.add(l.x(4096, 1024), l.x(4096, 1024)) for _ in range(4)])) == 1
+    l = FarList()
+    assert len(l.steps([l.add(l.x(4096, 1024), l.x(4096, 1024)) for _ in range(2)])) == 2
+    l = FarList()
+    y = l.concat(l.concat(l.x(20000, 256), l.x(20000, 256), 0), l.x(20000, 256), 0)
+    z = l.scale(l.x(8, 64), 2.0)
+    assert sorted(len(s) for s in l.steps([y, z])) == [1, 2]
+    l = FarList()
+    y = l.concat(l.concat(l.x(200, 256), l.x(200, 256), 0), l.x(200, 256), 0)
+    z = l.scale(l.x(8, 64), 2.0)
+    assert [len(s) for s in l.steps([y, z])] == [3]
+
+
+def test_large_launches_stay_in_the_lists_order():
+    l = FarList()
+    a = l.scale(l.x(8000, 512), 2.0)
+    b = l.scale(a, 2.0)
+    c = l.scale(l.x(8000, 512), 2.0)
+    assert l.steps([b, c, a]) == [[0], [1], [2]]

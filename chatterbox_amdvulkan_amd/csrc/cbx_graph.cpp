@@ -1825,7 +1825,7 @@ struct Scheduler {
             // (what no number of others makes worth sharing stays where it is: in
             // the list's order, its operands may still be in cache)
             if (link && from > 0 && steps[from - 1].kind == kStepRows && steps[from - 1].n < kStepMax &&
-                follows(from - 1, f.link)) {
+                chain_pays(3, f.link) && follows(from - 1, f.link)) {
                 to = from - 1;
                 info[to].link = f.link;
                 f.elts = 0;
@@ -1855,8 +1855,8 @@ struct Scheduler {
     }
 
     // The steps with those launches taken out of their step again, each into
-    // one of its own, that are the faster alone (a group's launches do not
-    // depend on each other).
+    // one of its own, that are the faster alone: a step's launches do not
+    // depend on each other, or (a chain's) run in their order.
     std::vector<Step>& settled() {
         std::vector<Step> out;
         out.reserve(steps.size());
@@ -1868,7 +1868,9 @@ struct Scheduler {
         };
         for (size_t q = 0; q < steps.size(); q++) {
             const Step& s = steps[q];
-            if (s.n > 1 && s.kind == kStepElt) {
+            if (s.n > 1 && s.kind == kStepRows && !chain_pays(s.n, info[q].link)) {
+                for (int32_t m = 0; m < s.n; m++) alone(s, m, 1);
+            } else if (s.n > 1 && s.kind == kStepElt) {
                 // entries: a launch, or a run of concats (the launches whose
                 // floats are counted with their first's)
                 auto entry = [&](int32_t m) {
@@ -1911,6 +1913,21 @@ struct Scheduler {
     int64_t most(size_t i, bool four) const {
         const int64_t small = int64_t{2048} * st->n_cu;
         return !four ? small : full[i] ? int64_t{1} << 26 : 2 * small;
+    }
+
+    // A chain keeps one row a workgroup, a launch of its own four once there
+    // are many: the chain pays while the launches are bound by their start,
+    // and further the more launches (and row loads) it saves.  Measured on 256
+    // CUs (us, one by one / chained): two launches (a LayerNorm and the add
+    // after it) 500 x 1024 9.1 / 7.8, 2000 x 1024 15.1 / 17.9, 24000 x 1024 96
+    // / 172, 1000 x 512 9.3 / 8.6, 3000 x 512 12.9 / 13.8, 2000 x 256 9.3 / 8.3,
+    // 6000 x 256 13.0 / 14.4; three with one LayerNorm among them 2000 x 1024
+    // 18.9 / 19.3, 8000 x 80 12.9 / 14.3; four (residual joins with their
+    // LayerNorms) 2000 x 1024 38.3 / 37.5, 4000 x 1024 62.4 / 68.4, 3000 x 512
+    // 28.8 / 23.3, 6000 x 256 29.2 / 25.5.
+    bool chain_pays(int32_t n, const LinkT& l) const {
+        const int64_t cu = st->n_cu;
+        return n == 2 ? l.nr <= 8 * cu && l.nr * l.ne0 <= 2560 * cu : l.nr <= 24 * cu && l.nr * l.ne0 <= 6144 * cu;
     }
 };
 

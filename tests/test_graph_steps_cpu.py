@@ -315,6 +315,30 @@ def test_group_of_whole_sums_and_concat_runs():
     assert [len(s) for s in l.steps([y, z])] == [3]
 
 
+@pytest.mark.parametrize("rows", [1 << 26, 1 << 28])
+def test_chain_of_more_rows_than_a_grid_takes(rows):
+    """A chain takes at least 64 work-items a row, so under 2^26 rows; the
+    launches alone take these."""
+    l = FarList()
+    j = l.add(l.x(rows, 4), l.add(l.x(rows, 4), l.x(4)))
+    y = l.scale(j, 2.0)
+    assert [p[0] for p in l.g.plan([j, y])] == [C.GL_BIAS_RESIDUAL, C.GL_SCALE]
+    assert [len(s) for s in l.steps([j, y])] == [1, 1]
+
+
+@pytest.mark.parametrize("T,D,n,chained", [(640, 1024, 2, True), (1000, 1024, 2, False), (1280, 512, 2, True),
+                                           (2000, 512, 2, False), (2048, 256, 2, True), (2049, 80, 2, False),
+                                           (1536, 1024, 4, True), (1537, 1024, 4, False), (6144, 80, 4, True),
+                                           (6145, 80, 4, False)])
+def test_chain_only_where_it_is_the_faster(T, D, n, chained):
+    l = FarList()
+    h, keep = l.x(T, D), []
+    for _ in range(n):
+        h = l.add(h, l.add(l.x(T, D), l.x(D)))
+        keep.append(l.layer_norm(h, l.x(D), l.x(D)))
+    assert [len(s) for s in l.steps(keep)] == ([n] if chained else [1] * n)
+
+
 def test_large_launches_stay_in_the_lists_order():
     l = FarList()
     a = l.scale(l.x(8000, 512), 2.0)

@@ -338,7 +338,8 @@ bool res_layer_fits(const ResLayer& l, int ch, const DeviceState* st) {
     const int64_t m = res_rows(ch);
     if (m == 0 || res_lds(l, ch, m) > 64 * 1024) return false;
     const int64_t tiles = res_tiles(l, m), k = l.k1 + l.k2, n_cu = st->n_cu;
-    if (tiles < 1 || tiles >= (int64_t{1} << 26)) return false;
+    // kResMax layers of this many tiles, 512 work-items each: under 2^32 a launch
+    if (tiles < 1 || tiles >= (int64_t{1} << 21)) return false;
     if (ch == 256 && k > 6) return k > 14 ? 3 * tiles >= 2 * n_cu : 3 * tiles >= n_cu;
     return (k > 14 ? 3 : 8) * tiles >= n_cu;
 }

@@ -345,3 +345,11 @@ def test_large_launches_stay_in_the_lists_order():
     b = l.scale(a, 2.0)
     c = l.scale(l.x(8000, 512), 2.0)
     assert l.steps([b, c, a]) == [[0], [1], [2]]
+
+
+@pytest.mark.parametrize("T,fused", [(1 << 20, True), (1 << 27, False)])
+def test_layer_of_more_tiles_than_a_grid_takes(T, fused):
+    """512 work-items a tile, three layers a launch: under 2^21 tiles each."""
+    l = FarList()
+    y, _ = l.layer(l.x(T, 256), 256, 3, 1)
+    assert ([len(s) for s in l.steps([y])] == [2]) == fused

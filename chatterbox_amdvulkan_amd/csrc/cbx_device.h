@@ -285,12 +285,12 @@ constexpr float kSinSmall = 65536.0f;
 
 // sin(x)^2 for |x| < 2^16.  q = round(x * 2/pi) as the low bits of a float
 // of magnitude 1.5 * 2^23 (one FMA; its low bit is q's parity).  Cody-Waite
-// reduction x = q*pi/2 + r with pi/2 split into two f32 parts P1 + P2:
-// x - q*P1 is exact (x and q*P1 are multiples of the last place of P1 or
-// finer, and the difference is under 1), the q*P2 correction rounds once in
-// its FMA, and the remaining q * (pi/2 - P1 - P2) is below 2^-33 (a third
-// part changes no error figure: 2.0e-8 rms and 1.1e-7 at most against 64
-// bits, with or without it, on |x| < 3 as on |x| < 65000); then the
+// reduction x = q*pi/2 + r with pi/2 split into three f32 parts P1 + P2 +
+// P3: x - q*P1 is exact (x and q*P1 are multiples of the last place of P1 or
+// finer, and the difference is under 1), the q*P2 and q*P3 corrections round
+// once each in their FMAs, and the remaining q * (pi/2 - P1 - P2 - P3) is
+// below 2^-57 (with two parts the relative error next to multiples of pi,
+// where r is small, is 1e-4 instead of 3e-7); then the
 // Taylor polynomial of sin r on |r| <= pi/4 (+ rounding slack): the first
 // omitted term is r^11/11! < 2.2e-9, under half an f32 ulp of the result.
 // sin(x)^2 = sin(r)^2 for even q, cos(r)^2 = 1 - sin(r)^2 for odd q (in one
@@ -301,6 +301,7 @@ __device__ __forceinline__ float sin_sq_small(float x) {
     const float q = qm - kRound;
     float r = fmaf(q, -0x1.921fb6p+0f, x);
     r = fmaf(q, 0x1.777a5cp-25f, r);
+    r = fmaf(q, 0x1.ee59dap-50f, r);
     const float r2 = r * r;
     float ps = fmaf(r2, 1.0f / 362880.0f, -1.0f / 5040.0f);
     ps = fmaf(ps, r2, 1.0f / 120.0f);

@@ -88,3 +88,20 @@ def test_snake_stage_shapes(cbx, oracle, shape):
     got = host(cbx.snake(dev(x), dev(a), dev(ai)))
     exp = oracle.snake(x, a, ai, nth=8)
     report("SNAKE", f"[{B},{Ch},{T}]", got, exp, x)
+
+
+def test_snake_sin_squared_near_multiples_of_pi(cbx):
+    """Snake's sin(x)^2 in relative terms where it is smallest: x + sin(x)^2 *
+    2^100, whose first term vanishes, at the f32 values next to k pi up to
+    2^16.  The reduced argument r (2^-27 at least) carries two roundings, 2^-24
+    of it each, and the rest of the split, 2^-57; the polynomial two more, all
+    of them twice in the square, which rounds once itself: under 16 * 2^-24."""
+    k = np.arange(1, 20861, dtype=np.float64)
+    x = (k * np.pi).astype(np.float32)
+    x = np.concatenate([x, np.nextafter(x, np.float32(0)), np.nextafter(x, np.float32(np.inf)), -x])
+    x = np.ascontiguousarray(x[np.abs(x) < 65536][:len(x) // 4 * 4].reshape(-1, 1).repeat(4, 1))
+    a, ai = np.ones(4, np.float32), np.full(4, 2.0 ** 100, np.float32)
+    got = host(cbx.snake(dev(x), dev(a), dev(ai))).astype(np.float64) / 2.0 ** 100
+    exp = np.sin(x.astype(np.float64)) ** 2
+    rel = np.abs(got - exp) / exp
+    assert rel.max() < 2.0 ** -20, f"largest relative error {rel.max():.3g}"

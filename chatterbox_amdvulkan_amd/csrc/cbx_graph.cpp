@@ -1598,14 +1598,34 @@ struct Scheduler {
     std::vector<int32_t> order, first;          // the tensors class by class; each class's first in it
     std::vector<int32_t> last_rd, last_wr;      // by class: the last step, or -1
     std::vector<int32_t> rd, wr;                // the current launch's classes
+    std::vector<int32_t> reads, writes;         // the tensors each planned launch reads and stores, launch i's
+    std::vector<int32_t> r0, w0;                // from r0[i] and w0[i] on
     std::vector<int64_t> floats;                // by planned launch: what its element-wise ops store
     std::vector<char> full;                     // one unactivated op of two whole operands
 
     void classes(int32_t n_t) {
+        // what no launch reads or stores (the launches' intermediates) and
+        // nothing keeps is in no class
+        std::vector<char> used(keep);
+        reads.reserve(6 * ls.size());
+        writes.reserve(2 * ls.size());
+        r0.reserve(ls.size() + 1);
+        w0.reserve(ls.size() + 1);
+        for (const cbx_glaunch& l : ls) {
+            r0.push_back(static_cast<int32_t>(reads.size()));
+            w0.push_back(static_cast<int32_t>(writes.size()));
+            if (l.kind == CBX_GL_VIEW) continue;
+            each_access(l, [&](int32_t i) { reads.push_back(i); }, [&](int32_t i) { writes.push_back(i); });
+        }
+        r0.push_back(static_cast<int32_t>(reads.size()));
+        w0.push_back(static_cast<int32_t>(writes.size()));
+        for (int32_t i : reads) used[static_cast<size_t>(i)] = 1;
+        for (int32_t i : writes) used[static_cast<size_t>(i)] = 1;
         std::vector<std::pair<Span, int32_t>> v;
         v.reserve(static_cast<size_t>(n_t));
         cls.assign(static_cast<size_t>(n_t), -1);
         for (int32_t i = 0; i < n_t; i++) {
+            if (!used[static_cast<size_t>(i)]) continue;
             const Span p = span_of(t[i]);
             if (p.hi > p.lo) v.push_back({p, i});
         }
@@ -1651,10 +1671,13 @@ struct Scheduler {
         }
     }
 
-    // Adds the classes that a launch reads (but for tensor `skip`) and stores
-    // to rd and wr.
-    void accesses(const cbx_glaunch& l, int32_t skip = -1) {
-        each_access(l, [&](int32_t s) { if (s != skip) touch(&rd, s); }, [&](int32_t d) { touch(&wr, d); });
+    // Adds the classes that planned launch i reads (but for tensor `skip`) and
+    // stores to rd and wr.
+    void accesses(size_t i, int32_t skip = -1) {
+        for (int32_t k = r0[i]; k < r0[i + 1]; k++) {
+            if (reads[static_cast<size_t>(k)] != skip) touch(&rd, reads[static_cast<size_t>(k)]);
+        }
+        for (int32_t k = w0[i]; k < w0[i + 1]; k++) touch(&wr, writes[static_cast<size_t>(k)]);
     }
 
     // Whether tensor d's bytes, as stored before planned launch `from`, are
@@ -1674,13 +1697,13 @@ struct Scheduler {
             }
             return false;
         };
-        bool seen = false;
         for (size_t i = from; i < ls.size() && !live.empty(); i++) {
-            if (ls[i].kind == CBX_GL_VIEW) continue;
-            each_access(ls[i], [&](int32_t s) { seen = seen || meets(s); }, [](int32_t) {});
-            if (seen) return true;
-            each_access(ls[i], [](int32_t) {}, [&](int32_t w) {
-                if (!meets(w) || !is_contiguous(&t[w])) return;
+            for (int32_t k = r0[i]; k < r0[i + 1]; k++) {
+                if (meets(reads[static_cast<size_t>(k)])) return true;
+            }
+            for (int32_t k = w0[i]; k < w0[i + 1]; k++) {
+                const int32_t w = writes[static_cast<size_t>(k)];
+                if (!meets(w) || !is_contiguous(&t[w])) continue;
                 const Span p = span_of(t[w]);
                 std::vector<Span> left;
                 for (const Span& b : live) {
@@ -1688,7 +1711,7 @@ struct Scheduler {
                     if (p.hi < b.hi) left.push_back({std::max(b.lo, p.hi), b.hi});
                 }
                 live.swap(left);
-            });
+            }
         }
         for (; m != end; m++) {
             if (keep[static_cast<size_t>(*m)] && meets(*m)) return true;
@@ -1767,6 +1790,8 @@ struct Scheduler {
 
     std::vector<Step>& run(int32_t n_t) {
         classes(n_t);
+        steps.reserve(ls.size());
+        info.reserve(ls.size());
         floats.assign(ls.size(), 0);
         full.assign(ls.size(), 0);
         for (size_t i = 0; i < ls.size();) {
@@ -1778,7 +1803,7 @@ struct Scheduler {
             s.li[s.n++] = static_cast<int32_t>(at);
             rd.clear();
             wr.clear();
-            accesses(l);
+            accesses(at);
             int ch = 0;
             SoftMaxCall sc;
             EltOp eo[kConcatMax + 1];
@@ -1790,7 +1815,7 @@ struct Scheduler {
                 // conv1's output is neither stored nor read (that tensor: what
                 // else its bytes' class holds, x or the residual, is read)
                 wr.clear();
-                accesses(ls[i++], nd[l.first_node + l.n_nodes - 1].dst);
+                accesses(i++, nd[l.first_node + l.n_nodes - 1].dst);
             } else if (l.kind == CBX_GL_CONCAT) {
                 while (s.n < kConcatMax && appends(i)) s.li[s.n++] = static_cast<int32_t>(i++);
                 // the longest run of them that is plain copies
@@ -1858,6 +1883,9 @@ struct Scheduler {
     // one of its own, that are the faster alone: a step's launches do not
     // depend on each other, or (a chain's) run in their order.
     std::vector<Step>& settled() {
+        bool shared = false;   // launches that might
+        for (const Step& s : steps) shared = shared || (s.n > 1 && (s.kind == kStepRows || s.kind == kStepElt));
+        if (!shared) return steps;
         std::vector<Step> out;
         out.reserve(steps.size());
         auto alone = [&](const Step& s, int32_t m, int32_t n) {
@@ -1934,9 +1962,10 @@ struct Scheduler {
 std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd, int32_t n,
                            const std::vector<cbx_glaunch>& ls, const int32_t* keep, int32_t n_keep,
                            const DeviceState* st) {
-    if (!st) {   // the launches report it
+    if (!st || ls.size() == 1) {   // without a state the launches report it
         std::vector<Step> one;
         for (size_t i = 0; i < ls.size(); i++) {
+            if (ls[i].kind == CBX_GL_VIEW) continue;
             Step s;
             s.li[s.n++] = static_cast<int32_t>(i);
             one.push_back(s);
@@ -1944,7 +1973,7 @@ std::vector<Step> schedule(const cbx_tensor* t, int32_t n_t, const cbx_gnode* nd
         return one;
     }
     Scheduler s{t, nd, ls, st, std::vector<int32_t>(static_cast<size_t>(n_t), 0),
-                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
+                std::vector<char>(static_cast<size_t>(n_t), 0), {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
     for (int32_t k = 0; k < n_keep; k++) s.keep[static_cast<size_t>(keep[k])] = 1;
     for (int32_t i = 0; i < n; i++) {
         for (int32_t q : nd[i].src) {

@@ -353,3 +353,23 @@ def test_layer_of_more_tiles_than_a_grid_takes(T, fused):
     l = FarList()
     y, _ = l.layer(l.x(T, 256), 256, 3, 1)
     assert ([len(s) for s in l.steps([y])] == [2]) == fused
+
+
+def test_unstored_intermediates_are_no_conflicts():
+    """A result that no launch stores (the first layer's im2col) may lie over
+    what two independent layers store: they share a launch all the same."""
+    ch, T = 64, 12000
+    l = HostList()
+    ys = [l.layer(l.x(T, ch), ch, 3, 1)[0] for _ in range(2)]
+    buf = torch.empty(2 * ch * T + 64)
+    for k, y in enumerate(ys):
+        l.place(y, buf, k * ch * T)
+    assert [len(s) for s in l.steps(ys)] == [4]
+    col = l.g.nodes[[i for i, n in enumerate(l.g.nodes) if n.op == C.GOP_IM2COL][0]].dst
+    scratch = buf.view(torch.float16)[:3 * ch * T].view(l.at(col).shape)
+    l.g.rebind(col, scratch)
+    assert [len(s) for s in l.steps(ys)] == [4]
+    # something that a launch does store there is a conflict
+    over = l.scale(l.t(buf[:2 * ch * T].view(2 * T, ch)), 2.0)
+    steps = l.steps(ys + [over])
+    assert step_of(l, ys + [over], over) > max(step_of(l, ys + [over], y) for y in ys) and len(steps) == 2

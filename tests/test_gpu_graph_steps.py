@@ -38,10 +38,12 @@ class Lists:
         self.keep.append(i)
         return i
 
-    def check(self, replays=3):
+    def check(self, steps, replays=3):
+        """steps: how many kernels the list is issued as on 256 CUs."""
         g, before = self.b.g, [t.clone() for t in self.made]
         T, N, _ = g._arrays(self.keep)
         plan = g.plan(self.keep)
+        assert len(g.steps(self.keep)) == len(g.steps(self.keep, 256)) == steps
         for p in plan:
             rc = C.load().cbx_graph_launch(T, len(g._descs), N, len(g.nodes), ctypes.byref(C.GLaunch(*p)), C._stream())
             assert rc == C.OK, C.last_error()
@@ -89,12 +91,13 @@ def test_elementwise(cbx, T, D):
     y = l.k(b.scale(l.x(T, D), 2.0))
     y = l.k(b.add(y, l.x(T, D)))
     l.k(b.unary(y, C.TANH))
-    l.check()
+    l.check(3)
 
 
-@pytest.mark.parametrize("parts,kept", [((4, 4), ()), ((8, 80, 4), ()), ((80, 80, 80, 80), ()), ((256, 4, 12, 8, 16), ()),
-                                        ((4,) * 9, ()), ((80, 80, 80, 80), (1,)), ((80, 3, 5, 80), ())])
-def test_concats(cbx, parts, kept):
+@pytest.mark.parametrize("parts,kept,steps", [((4, 4), (), 1), ((8, 80, 4), (), 1), ((80, 80, 80, 80), (), 1),
+                                              ((256, 4, 12, 8, 16), (), 1), ((4,) * 9, (), 2),
+                                              ((80, 80, 80, 80), (1,), 2), ((80, 3, 5, 80), (), 3)])
+def test_concats(cbx, parts, kept, steps):
     """Runs of concats along dim 0: only the last result is stored unless a
     caller keeps one between; odd widths run as they are."""
     l = Lists(sum(parts))
@@ -106,11 +109,12 @@ def test_concats(cbx, parts, kept):
             l.k(y)
     l.k(y)
     l.k(b.scale(l.x(T, 64), 3.0))
-    l.check()
+    l.check(steps)
 
 
-@pytest.mark.parametrize("heads,q,kv", [(8, 125, 125), (8, 250, 250), (16, 1, 257), (8, 300, 300), (3, 7, 1100), (8, 500, 77)])
-def test_softmaxes(cbx, heads, q, kv):
+@pytest.mark.parametrize("heads,q,kv,steps", [(8, 125, 125, 3), (8, 250, 250, 3), (16, 1, 257, 3), (8, 300, 300, 3),
+                                              (3, 7, 1100, 10), (8, 500, 77, 3)])
+def test_softmaxes(cbx, heads, q, kv, steps):
     l = Lists(heads * q + kv)
     b = l.b
     for n in range(5):
@@ -122,7 +126,7 @@ def test_softmaxes(cbx, heads, q, kv):
     # another length with the same rows, and one that reads a softmax
     l.k(b.soft_max(b.scale(l.x(heads, q, kv + 4), 0.5)))
     l.k(b.soft_max(b.scale(l.keep[0], 2.0)))
-    l.check()
+    l.check(steps)
 
 
 def ln(l, x, eps=1e-5):
@@ -131,10 +135,11 @@ def ln(l, x, eps=1e-5):
 
 
 # one wave a row, several, one row to several rounds of rows, more links than
-# a chain holds
-@pytest.mark.parametrize("T,D,n", [(1, 1024, 30), (3, 4, 3), (500, 256, 4), (125, 512, 5), (250, 260, 2), (2100, 512, 3),
-                                   (2100, 1024, 2), (7, 768, 4), (20, 1028, 2)])
-def test_row_chain(cbx, T, D, n):
+# a chain holds; rows longer than a chain takes, and more floats than one is
+# the faster for
+@pytest.mark.parametrize("T,D,n,steps", [(1, 1024, 30, 4), (3, 4, 3, 3), (500, 256, 4, 3), (125, 512, 5, 3), (250, 260, 2, 3),
+                                         (2100, 512, 3, 5), (2100, 1024, 2, 13), (7, 768, 4, 3), (20, 1028, 2, 11)])
+def test_row_chain(cbx, T, D, n, steps):
     l = Lists(T + D + n)
     b = l.b
     mask = b.t((torch.rand((T, 1), generator=l.gen, device="cuda") > 0.2).float())
@@ -153,12 +158,13 @@ def test_row_chain(cbx, T, D, n):
         l.k(b.unary(b.add(l.x(T, 2 * D), l.x(2 * D)), C.GELU))
         h = h2
     l.k(b.add(h, b.add(l.x(T, D), l.x(D))))
-    l.check()
+    l.check(steps)
 
 
 def test_shared_buffers(cbx):
     """Results that take over the bytes of earlier tensors (in place, or a
-    buffer used again, whole or in part): the order of the list holds."""
+    buffer used again, whole or in part): the order of the list holds, while
+    the launches between them that touch none of it share one kernel."""
     T, D = 64, 256
     l = Lists(11)
     b, g = l.b, l.b.g
@@ -172,25 +178,34 @@ def test_shared_buffers(cbx):
         g.node(C.GOP_ADD, dst, (x, y))
         return dst
 
+    def aside():
+        l.k(b.scale(l.x(T, D), 1.5))
+
     n = T * D
     a = add(at(0), l.x(T, D), l.x(T, D))
     c = l.k(b.scale(a, 2.0))
+    aside()
     d = add(at(0), l.x(T, D), l.x(T, D))              # over a, read above
     l.k(b.mul(d, c))
+    aside()
     e = add(at(n // 2), l.x(T, D), l.x(D))            # half over d
     l.k(ln(l, e))
+    aside()
     f = add(e, e, l.x(T, D))                          # in place
     h = l.k(ln(l, f))
+    aside()
     s = add(at(n), f, h)
     l.k(ln(l, s))
+    aside()
     s2 = add(at(n), s, l.x(T, D))                     # the sum in place, its norm next
     l.k(ln(l, s2))
     l.k(b.soft_max(b.scale(s2, 0.5)))
+    aside()
     add(at(n), l.x(T, D), l.x(T, D))                  # over s2 after its readers
     l.k(at(0))
     l.k(at(n))
     l.k(at(n // 2))
-    l.check()
+    l.check(10)
 
 
 def test_misaligned_rows_run_alone(cbx):
@@ -206,7 +221,7 @@ def test_misaligned_rows_run_alone(cbx):
         l.k(b.scale(x, 2.0))
     l.k(b.soft_max(b.scale(x, 0.3)))
     l.k(b.soft_max(b.scale(l.x(T, D), 0.3)))
-    l.check()
+    l.check(6)
 
 
 def test_update_moves_between_steps(cbx):

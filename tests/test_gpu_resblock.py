@@ -79,7 +79,9 @@ def add_layer(b, x, p, d, convs):
     return b.sublayer(x, {n: b.t(t) for n, t in p.items()}, d, *cw)
 
 
-def replay(b, keep, convs, n=2):
+def replay(b, keep, convs, steps, n=2):
+    """steps: how many kernels the list is issued as on 256 CUs."""
+    assert len(b.g.steps(keep)) == steps
     ex = b.g.capture(keep)
     try:
         for _ in range(n):
@@ -114,7 +116,7 @@ def test_layer(cbx, ch, K, d, T):
     p, x, convs = params(g, ch, K), rnd(g, T, ch), []
     b = NodeList(new)
     y = add_layer(b, b.t(x), p, d, convs)
-    got, = replay(b, [y], convs)
+    got, = replay(b, [y], convs, steps=1)
     ref, bound = layer(x.double(), p, d)
     check(got, ref, bound, f"{ch} x {T} K {K} d {d}")
 
@@ -137,15 +139,18 @@ def test_three_blocks_and_their_sum(cbx, ch, T):
             rr, nb = layer(rr.float().double(), p, d)
             # the incoming difference through both convs of this layer
             rb = nb if d == 1 else rb + nb + 4 * conv(conv(rb, p["w1"].double().abs(), d), p["w2"].double().abs(), 1)
+        if total is None:
+            first, first_ref, first_bound = r, rr, rb
         total = r if total is None else b.add(total, r)
         ref = rr if ref is None else ref + rr
         bound = rb if bound is None else bound + rb
     y = b.scale(total, 1.0 / 3.0)
-    got, = replay(b, [y], convs)
-    d = (got - ref / 3.0).abs()
-    assert torch.isfinite(got).all() and not (d > bound).any()
-    # an f16 operand flipped in layer one flips more in layer two: a few 1e-4
-    assert float((got - ref / 3.0).norm() / (ref / 3.0).norm()) < 1e-3
+    # the first layers share a launch; the sum runs through the second ones
+    outs = replay(b, [first, y], convs, steps=4)
+    for got, exp, bd in zip(outs, (first_ref, ref / 3.0), (first_bound, bound)):
+        assert torch.isfinite(got).all() and not ((got - exp).abs() > bd).any()
+        # an f16 operand flipped in layer one flips more in layer two: a few 1e-4
+        assert float((got - exp).norm() / exp.norm()) < 1e-3
 
 
 def test_large_arguments(cbx):
@@ -158,7 +163,7 @@ def test_large_arguments(cbx):
     p, x, convs = params(g, ch, K, alpha=2.0 ** 18), rnd(g, T, ch), []
     b = NodeList(new)
     y = add_layer(b, b.t(x), p, d, convs)
-    got, = replay(b, [y], convs)
+    got, = replay(b, [y], convs, steps=1)
     ref, bound = layer(x.double(), p, d)
     free = torch.zeros(T, ch, dtype=torch.float64, device="cuda")
     free[:, ::7] = 2.0 ** -14
@@ -174,7 +179,7 @@ def test_infinite_input_stays_in_its_reach(cbx):
     x[t, 9] = float("inf")
     b = NodeList(new)
     y = add_layer(b, b.t(x), p, d, convs)
-    got, = replay(b, [y], convs)
+    got, = replay(b, [y], convs, steps=1)
     bad = ~torch.isfinite(got).all(1)
     lo, hi = t - 3 * d - 3, t + 3 * d + 3
     assert not bad[:lo].any() and not bad[hi + 1:].any() and bool(bad[t])
@@ -202,6 +207,7 @@ def test_layers_the_launch_leaves_alone(cbx, how):
     if how == "in place":
         dst = b.t(x)
         b.g.nodes[-1].dst = dst
+        assert len(b.g.steps([dst])) == 2
         ex = b.g.capture([dst])
         ex.launch()
         torch.cuda.synchronize()
@@ -210,6 +216,45 @@ def test_layers_the_launch_leaves_alone(cbx, how):
         for c in convs:
             c.close()
     else:
-        got = replay(b, keep, convs)[-1]
+        got = replay(b, keep, convs, steps=2)[-1]
     ref, bound = layer(x0.double(), p, d)
     check(got, ref, bound, how)
+
+
+@pytest.mark.parametrize("ch,T", [(64, 126 * 60 + 5), (128, 62 * 60 + 5)])
+def test_layers_over_buffers_used_again(cbx, ch, T):
+    """Layer 2 reads layer 1's result, beside which its own first conv's output
+    lies in one arena that an earlier tensor spans; a later launch writes over
+    that result."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(ch + 1)
+    p1, p2, x, convs = params(g, ch, 3), params(g, ch, 3), rnd(g, T, ch), []
+    arena = torch.empty(2 * T * ch, device="cuda")
+    b = NodeList(new)
+    span = b.t(arena.view(2 * T, ch))
+    dead = b.scale(span, 2.0)
+    y1 = add_layer(b, b.t(x), p1, 1, convs)
+    b.g.rebind(y1, arena[:T * ch].view(T, ch))
+    n = len(b.g.nodes)
+    y2 = add_layer(b, y1, p2, 3, convs)
+    sin = [i for i in range(n, len(b.g.nodes)) if b.g.nodes[i].op == C.GOP_UNARY and b.g.nodes[i].iparam == C.SIN][1]
+    b.g.rebind(b.g.nodes[sin - 1].src[0], arena[T * ch:].view(T, ch))
+    over = b.scale(b.t(x), 3.0)
+    b.g.rebind(over, arena[:T * ch].view(T, ch))
+    assert [len(s) for s in b.g.steps([dead, y2, over])] == [1, 2, 2, 1]
+    ex = b.g.capture([dead, y2, over])
+    for _ in range(2):
+        arena.fill_(1.0)
+        b.at(y2).fill_(float("nan"))
+        ex.launch()
+        torch.cuda.synchronize()
+        r1, bound1 = layer(x.double(), p1, 1)
+        r2, bound2 = layer(r1.float().double(), p2, 3)
+        w1 = p2["w1"].double().abs()
+        bound = bound1 + bound2 + 4 * conv(conv(bound1, w1, 3), p2["w2"].double().abs(), 1)
+        got = b.at(y2).double()
+        assert torch.isfinite(got).all() and not ((got - r2).abs() > bound).any()
+        assert torch.equal(b.at(over), x * 3.0) and bool((b.at(dead) == 2.0).all())
+    ex.close()
+    for c in convs:
+        c.close()

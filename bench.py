@@ -600,7 +600,7 @@ def graph_exec_costs(C, torch, base, n_blocks, s, calls=100):
     def compute():
         check_rc(C, L.cbx_graph_compute(Tn, len(g._descs), Nn, len(g.nodes), Kn, len(keep), s, ctypes.byref(n)))
 
-    res = {"launches": ex.n_launches}
+    res = {"launches": ex.n_launches, "kernels": len(g.steps(keep))}
     for name, f in (("compute", compute), ("exec", lambda: ex.launch(s))):
         for _ in range(5):
             f()
@@ -614,12 +614,16 @@ def graph_exec_costs(C, torch, base, n_blocks, s, calls=100):
         e1.record()
         torch.cuda.synchronize()
         res[name] = {"host_us": host, "device_us": e0.elapsed_time(e1) * 1000.0 / calls}
-    # re-pointing the exec at the list (the next step of a loop; here the same
-    # buffers, so the same launches: taken in place) against capturing anew
+    # re-pointing the exec at the list with other buffers for a matmul's output
+    # (the next step of a loop: the same launches, taken in place) against
+    # capturing anew; three in turn, so that neither of the exec's two
+    # instantiations holds the next one already
+    bufs = [base["fc_mm"], torch.empty_like(base["fc_mm"]), torch.empty_like(base["fc_mm"])]
     ip = ctypes.c_int32(0)
     upd = new = 0.0
     reps = max(1, calls // 5)
-    for _ in range(reps):
+    for k in range(reps):
+        Tn[T["fc_mm"]].data = bufs[(k + 1) % 3].data_ptr()
         torch.cuda.synchronize()
         tm = time.perf_counter()
         check_rc(C, L.cbx_graph_exec_update(ex.handle, Tn, len(g._descs), Nn, len(g.nodes), Kn, len(keep),
@@ -748,7 +752,7 @@ def bench_t3_token(C, W, torch, reps=200, tokens=64):
     st.set_token(17, n0)
     ex = st.graph.capture(st.keep)
     s = cur_stream(torch)
-    out = {"launches": ex.n_launches, "blocks": st.n_blocks, "n_past": n0,
+    out = {"launches": ex.n_launches, "kernels": len(st.graph.steps(st.keep)), "blocks": st.n_blocks, "n_past": n0,
            "bytes_per_token": W.t3_token_bytes(st.n_blocks, n0)}
     for _ in range(10):
         ex.launch(s)
@@ -761,7 +765,7 @@ def bench_t3_token(C, W, torch, reps=200, tokens=64):
     torch.cuda.synchronize()
     dev_us = e0.elapsed_time(e1) * 1000.0 / reps
     out["exec_replay_us_per_token"] = dev_us
-    out["exec_replay_us_per_launch"] = dev_us / ex.n_launches
+    out["exec_replay_us_per_kernel"] = dev_us / out["kernels"]
     # plan + launch every token (no graph)
     for _ in range(3):
         st.graph.compute(st.keep)
@@ -851,7 +855,8 @@ def bench_cfm_estimator(C, torch, T=500, reps=20):
             if p[0] != C.GL_VIEW:
                 kinds[names[p[0]]] = kinds.get(names[p[0]], 0) + 1
         out = {"reference_sequence": f"cfm_decoder.cpp:395-558, T_mel {T}, 14 resnet blocks, 56 transformer blocks",
-               "launches": ex.n_launches, "launches_by_kind": kinds, "bytes_per_call": nbytes}
+               "launches": ex.n_launches, "kernels": len(e.graph.steps(e.keep)), "launches_by_kind": kinds,
+               "bytes_per_call": nbytes}
         for _ in range(3):
             ex.launch(s)
         torch.cuda.synchronize()
@@ -863,7 +868,7 @@ def bench_cfm_estimator(C, torch, T=500, reps=20):
         torch.cuda.synchronize()
         dev_us = e0.elapsed_time(e1) * 1000.0 / reps
         out["exec_replay_us_per_call"] = dev_us
-        out["exec_replay_us_per_launch"] = dev_us / ex.n_launches
+        out["exec_replay_us_per_kernel"] = dev_us / out["kernels"]
         out["GBps"] = nbytes / (dev_us * 1e-6) / 1e9
         ex.close()
         for _ in range(2):
@@ -897,8 +902,8 @@ def bench_node_list(C, torch, e, ref, reps):
     for p in plan:
         if p[0] != C.GL_VIEW:
             kinds[names[p[0]]] = kinds.get(names[p[0]], 0) + 1
-    out = {"reference_sequence": ref, "launches": ex.n_launches, "launches_by_kind": kinds,
-           "bytes_per_call": nbytes}
+    out = {"reference_sequence": ref, "launches": ex.n_launches, "kernels": len(e.graph.steps(e.keep)),
+           "launches_by_kind": kinds, "bytes_per_call": nbytes}
     for _ in range(3):
         ex.launch(s)
     torch.cuda.synchronize()
@@ -910,7 +915,7 @@ def bench_node_list(C, torch, e, ref, reps):
     torch.cuda.synchronize()
     dev_us = e0.elapsed_time(e1) * 1000.0 / reps
     out["exec_replay_us_per_call"] = dev_us
-    out["exec_replay_us_per_launch"] = dev_us / ex.n_launches
+    out["exec_replay_us_per_kernel"] = dev_us / out["kernels"]
     out["GBps"] = nbytes / (dev_us * 1e-6) / 1e9
     ex.close()
     for _ in range(2):
@@ -984,7 +989,8 @@ def bench_hift_decode(C, torch, T_mel=500, reps=10):
                 kinds[names[p[0]]] = kinds.get(names[p[0]], 0) + 1
         out = {"reference_sequence": f"hift_vocoder.cpp:613-749, T_mel {T_mel} "
                                      f"(stages of {e.stage_frames[0]}, {e.stage_frames[1]}, {e.stage_frames[2]} frames)",
-               "launches": ex.n_launches, "launches_by_kind": kinds, "conv_flop_per_decode": flops}
+               "launches": ex.n_launches, "kernels": len(e.graph.steps(e.keep)), "launches_by_kind": kinds,
+               "conv_flop_per_decode": flops}
         for _ in range(2):
             ex.launch(s)
         torch.cuda.synchronize()

@@ -1234,9 +1234,10 @@ int run(const cbx_tensor* t, const cbx_gnode* nd, int32_t n_nodes, const cbx_gla
 // each other, and chains of dependent row launches (k_group.hip).  A launch
 // joins the earliest step of its kind that follows every step it conflicts
 // with, by the bytes it reads and stores, so the values are those of the
-// launches in their order.  A ResBlock layer's conv1 output is the one
-// planned store a step leaves out, under the terms of a chain's
-// intermediates: nothing else reads it and the caller does not keep it.
+// launches in their order.  Two planned stores are left out: a ResBlock
+// layer's conv1 output, and the results of a run of concats but its last.
+// The next launch alone reads them, the caller does not keep them, and
+// their bytes are not read or kept under another descriptor.
 enum { kStepOne = 0, kStepLayers, kStepElt, kStepSoftMax, kStepRows };
 constexpr int kStepMax = 48;
 static_assert(kStepMax <= kEltMax && kStepMax <= kSoftMaxGroup && kStepMax <= kChainMax && 2 * kResMax <= kStepMax, "");

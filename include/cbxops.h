@@ -786,9 +786,11 @@ int cbx_graph_launch(const cbx_tensor* tensors, int32_t n_tensors,
  * *n_launches (may be NULL) gets the number of planned launches run.  They
  * are issued as fewer kernels where several can share one (independent
  * element-wise launches or softmaxes, chains of row launches, ResBlock
- * layers): the kept tensors are those of the launches in their order, a
- * ResBlock layer's first conv output that nothing else reads and keep does
- * not name may stay unstored.                                              */
+ * layers): the kept tensors are those of the launches in their order.  A
+ * ResBlock layer's first conv output, and the results of a run of concats
+ * but its last, may stay unstored when nothing but the next launch reads
+ * them and keep does not name them (also not under another descriptor of
+ * the same bytes).                                                         */
 int cbx_graph_compute(const cbx_tensor* tensors, int32_t n_tensors,
                       const cbx_gnode* nodes, int32_t n_nodes,
                       const int32_t* keep, int32_t n_keep,

@@ -213,6 +213,7 @@ def load() -> ctypes.CDLL:
         "cbx_graph_steps": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
                                 ctypes.POINTER(ctypes.c_int32), ctypes.c_int32, ctypes.c_int32,
                                 ctypes.POINTER(ctypes.c_int32), ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]),
+        "cbx_graph_exec_streams": (i, [vp]),
         "cbx_graph_launch": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,
                                  ctypes.POINTER(GLaunch), vp]),
         "cbx_graph_compute": (i, [P, ctypes.c_int32, ctypes.POINTER(GNode), ctypes.c_int32,

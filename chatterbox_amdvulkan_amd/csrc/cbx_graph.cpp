@@ -2521,13 +2521,6 @@ int cbx_graph_exec_update(cbx_graph_exec* exec, const cbx_tensor* tensors, int32
         std::vector<uint64_t> sig;
         std::vector<size_t> sig_at;
         signatures(tensors, nodes, ls, steps, &sig, &sig_at);
-        // the list the current instantiation already holds: nothing to set
-        const GraphInst& c = exec->inst[exec->cur];
-        if (c.indexed && c.steps == steps && c.sig == sig && c.ls.size() == ls.size()) {
-            if (n_launches) *n_launches = c.n_launches;
-            if (in_place) *in_place = 1;
-            return CBX_OK;
-        }
         // the instantiation to re-point is the one not replayed since the
         // last update: update_changed records first, waits for its replays
         // (issued before that update) and marks the current one's, then sets
@@ -2600,6 +2593,8 @@ int cbx_graph_exec_launch(cbx_graph_exec* exec, cbx_stream stream) {
     if (!seen) exec->launched.push_back(s);
     return CBX_OK;
 }
+
+int cbx_graph_exec_streams(const cbx_graph_exec* exec) { return exec ? static_cast<int>(exec->launched.size()) : 0; }
 
 void cbx_graph_exec_destroy(cbx_graph_exec* exec) {
     if (!exec) return;

@@ -369,3 +369,6 @@ enum { UNARY_LEAKY = 100 };
 extern "C" int cbx_graph_steps(const cbx_tensor* tensors, int32_t n_tensors, const cbx_gnode* nodes, int32_t n_nodes,
                                const int32_t* keep, int32_t n_keep, int32_t n_cu, int32_t* step, int32_t max_launches,
                                int32_t* n_launches);
+// For tests: the streams that the exec's next update or its destruction will
+// record an event on (those launched on since the last update).
+extern "C" int cbx_graph_exec_streams(const cbx_graph_exec* exec);

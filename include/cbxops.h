@@ -824,8 +824,8 @@ void cbx_graph_exec_destroy(cbx_graph_exec* exec);
  * loop: t3.cpp:604's decode graph with the position and the KV views of the
  * next token).  The list is planned and recorded again; when it gives the
  * same launches with other arguments (addresses, shapes, positions), the
- * instantiated graph takes them in place (*in_place = 1; a list it holds
- * already changes nothing), otherwise it is re-instantiated (*in_place = 0).  Stream-ordered: the exec's two
+ * instantiated graph takes them in place (*in_place = 1), otherwise it is
+ * re-instantiated (*in_place = 0).  Stream-ordered: the exec's two
  * instantiations take turns, and an update re-points the one not replayed
  * since the previous update, after waiting (on events recorded by that
  * update) for its replays -- all issued before the previous update -- and

@@ -579,3 +579,26 @@ def test_update_to_another_list(cbx):
     finally:
         ex.close()
         cache.close()
+
+
+def test_an_update_lets_go_of_every_stream(cbx):
+    """Streams need to exist until the next update only: an update marks the
+    replays on all of them, also when it changes nothing."""
+    x, y = torch.randn(64, 256, device="cuda"), torch.empty(64, 256, device="cuda")
+    g = cbx.Graph()
+    i, o = g.tensor(x), g.tensor(y)
+    g.node(cbx.GOP_SCALE, o, (i,), fparam=2.0)
+    ex = g.capture([o])
+    held = cbx.load().cbx_graph_exec_streams
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for scale in (2.0, 2.0, 2.0, 3.0, 3.0):
+        g.nodes[0].fparam = scale
+        assert ex.update(keep=[o]) is True
+        assert held(ex.handle) == 0
+        for s in streams:
+            ex.launch(s.cuda_stream)
+        assert held(ex.handle) == 2
+        torch.cuda.synchronize()
+        assert torch.equal(y, x * scale)
+    ex.close()
